@@ -226,16 +226,16 @@ int tla_matmul(tla_engine* e, float* out_dev, const void* w_dev, const float* x_
                int cols, int type);
 
 /* matmul() over a batch of n_tok vectors: out[t][rows] = W . x[t] (x
- * [n_tok][cols]).  3-64 vectors (F32, F16, Q8_0, Q4_0; F16 and F32 from
- * 2) run as one product that dequantises the weights in registers on the
- * fp32 matrix cores; from 65 vectors on (Q6_K from 16) as the split product:
- * x split into three bf16 pieces (an engine workspace of 6 bytes per
- * element, tokens padded to 64), weights dequantised in registers into exact
- * bf16 pieces, every product of pieces exact in the fp32 accumulator of the
- * bf16 matrix cores (K cut into ranges for small grids, their sums added in
- * order from a second workspace); fewer vectors (Q6_K: under 16) run as
- * groups of matrix-vector products.  fp32 accumulation throughout: equal to
- * the reference to fp32 rounding.  Used for the prompt's projections. */
+ * [n_tok][cols]).  From 3 vectors on (F16 and F32 from 2, Q6_K from 8) one
+ * split product: x split into three bf16 pieces, weights dequantised in
+ * registers into exact bf16 pieces, every product of pieces exact in the fp32
+ * accumulator of the bf16 matrix cores; up to 16 vectors, or for few rows,
+ * x is split by the product itself, else by a launch before it into an engine
+ * workspace of 6 bytes per element (tokens padded to 64), and rows of more than
+ * 2048 columns are cut into ranges whose sums are added in order from a
+ * second workspace.  Fewer vectors run as groups of matrix-vector products.
+ * fp32 accumulation throughout: equal to the reference to fp32 rounding.
+ * Used for the prompt's projections. */
 int tla_matmul_batch(tla_engine* e, float* out_dev, const void* w_dev, const float* x_dev, int rows,
                      int cols, int n_tok, int type);
 
@@ -358,10 +358,9 @@ int tla_forward(tla_engine* e, const tla_model* m, float* key_cache_dev, float* 
  * token's logits (the ones generate() samples from).  The KV cache ends as
  * after n_tok forward() calls (to fp32 rounding: the attention sums are
  * grouped differently).  Engine memory it keeps for later calls: the split
- * product's workspaces, for prompts past 64 tokens (or with a Q6_K layer
- * matrix past 15): 6 bytes per token (padded to 64) and column of the
- * widest product input (TinyLlama, 512 tokens: 17 MB), and partial sums of
- * at most a few MB. */
+ * product's workspaces, 6 bytes per token (padded to 64) and column of the
+ * widest product inputs, n_embd and n_ff (TinyLlama, 512 tokens: 24 MB), and
+ * partial sums of 4 bytes per token, row and 2048 columns of W_down (12 MB). */
 int tla_prefill_forward(tla_engine* e, const tla_model* m, float* key_cache_dev,
                         float* value_cache_dev, const int* tokens_host, int n_tok, int pos0,
                         float* logits_dev);
@@ -438,15 +437,16 @@ enum tla_option {
     TLA_OPT_DECODE_GROUP = 2, /* kv heads per decode workgroup in the plan of one split
                                  length: 1, 2 or 4 (the other plan always takes 4);
                                  results do not depend on it */
-    TLA_OPT_STREAM_TILES = 3, /* batched products of 2-64 vectors: vectors per
-                                 workgroup in tiles of 16, 1 to 4; results do not
-                                 depend on it */
-    TLA_OPT_SPLIT_ROWS = 4,   /* batched products past 64 vectors (Q6_K: from 16):
-                                 16-row subtiles per wave, 1, 2 or 4 (0: per
-                                 shape); results do not depend on it */
+    TLA_OPT_STREAM_TILES = 3, /* batched products that keep their weights in registers:
+                                 token tiles of 16 per workgroup, at most, 1 to 4;
+                                 results do not depend on it */
+    TLA_OPT_SPLIT_ROWS = 4,   /* batched products: 16-row subtiles per workgroup
+                                 or wave, 1, 2 or 4 (0: per shape; at most what the
+                                 format allows); results do not depend on it */
     TLA_OPT_SPLIT_K = 5       /* the same products: ranges K is cut into, 1 to 64
-                                 (0: per shape; at most one per 32-column block);
-                                 results change by fp32 rounding only */
+                                 (0: per shape; at least one per 2048 columns, at
+                                 most one per 64; products that split x themselves
+                                 take one); results change by fp32 rounding only */
 };
 enum tla_decode_plan { TLA_PLAN_AUTO = 0, TLA_PLAN_ALIGNED = 1, TLA_PLAN_BALANCED = 2 };
 int tla_set_option(tla_engine* e, int option, long long value);

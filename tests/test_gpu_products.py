@@ -1,0 +1,75 @@
+"""The split products of several tokens at the edges of their tiles, against
+fp64: the direct product (up to 16 tokens, or few rows), the resident one
+(more tokens; K in one or several ranges) and the tiled one (past 192
+tokens).
+
+Tolerance: a row is an fp32 sum of exact products in another order than the
+reference's, |gpu - fp64| <= 1e-5 sum |w x| (test_gpu_proj.py)."""
+import numpy as np
+import pytest
+
+import quant_ref as Q
+from helpers import device_arrays, log
+
+pytestmark = pytest.mark.gpu
+
+TYPES = [(Q.F32, "f32"), (Q.F16, "f16"), (Q.Q4_0, "q4_0"), (Q.Q8_0, "q8_0"), (Q.Q6_K, "q6_k")]
+# direct: one token tile, remainders of rows and waves; resident: shares of
+# the tiles, K slices of 4 and 8 blocks, two K ranges with an uneven last one;
+# tiled: K ranges, token and row remainders
+SHAPES = [(17, 64, 3), (33, 320, 8), (4112, 256, 16), (9000, 512, 15), (4112, 1024, 17), (4200, 2048, 33),
+          (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250)]
+
+
+def rows_close(got, raw, x, t, rows, cols, tol, what):
+    """got [n][rows] against W . x[i] for every token i."""
+    w = Q.dequant(raw, t, rows, cols)
+    ref, scale = x.astype(np.float64) @ w.T, np.abs(x).astype(np.float64) @ np.abs(w).T
+    err = float(np.max(np.abs(got - ref) / (scale + 1e-30)))
+    log(f"    {what}: {err:.2e}")
+    assert err <= tol, what
+
+
+@pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("rows,cols,n", SHAPES)
+def test_product_edges(W, engines, t, name, rows, cols, n):
+    if t == Q.Q6_K and cols % 256:
+        pytest.skip("Q6_K rows are whole 256-weight super-blocks")
+    eng = engines(1, 64)
+    raw = W.make_weights(t, rows, cols, salt=rows + cols)
+    x = np.random.default_rng(n + rows).standard_normal((n, cols)).astype(np.float32)
+    with device_arrays() as track:
+        w, xd = track(eng.array(raw)), track(eng.array(x))
+        out = track(eng.array((n + 1, rows)))  # one row more: stays as it was
+        guard = np.full((n + 1, rows), 7.25, np.float32)
+        out.upload(guard)
+        log(f"  product {name} {rows}x{cols}, {n} tokens")
+        eng.matmul_batch(out.ptr, w.ptr, xd.ptr, rows, cols, n, t)
+        got = out.download()
+    assert np.array_equal(got[n], guard[n])
+    rows_close(got[:n], raw, x, t, rows, cols, 1e-5, f"{name} {rows}x{cols} x {n}")
+
+
+@pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("n,rows", [(9, 48), (40, 4128)])
+def test_product_infinities(W, engines, t, name, n, rows):
+    """A token with an infinity, one with the largest float and one with a NaN
+    give what fp32 products give (the bf16 pieces of an infinity alone would
+    cancel to NaN); the other tokens are untouched by them."""
+    eng = engines(1, 64)
+    cols = 256
+    raw = W.make_weights(t, rows, cols, salt=3)
+    x = np.random.default_rng(5).standard_normal((n, cols)).astype(np.float32)
+    x[0, 40], x[1, 7], x[2, 200] = np.inf, np.finfo(np.float32).max, np.nan
+    with device_arrays() as track:
+        w, xd, out = track(eng.array(raw)), track(eng.array(x)), track(eng.array((n, rows)))
+        eng.matmul_batch(out.ptr, w.ptr, xd.ptr, rows, cols, n, t)
+        got = out.download()
+    wf = Q.dequant(raw, t, rows, cols)
+    col = wf[:, 40]
+    assert np.array_equal(got[0][col > 0], np.full((col > 0).sum(), np.inf, np.float32))
+    assert np.array_equal(got[0][col < 0], np.full((col < 0).sum(), -np.inf, np.float32))
+    assert np.isnan(got[0][col == 0]).all()
+    assert np.isnan(got[2]).all()
+    keep = [1] + list(range(3, n))
+    rows_close(got[keep], raw, x[keep], t, rows, cols, 1e-5, f"{name} finite tokens")

@@ -126,6 +126,8 @@ struct tla_engine {
     size_t fwd_bytes = 0;
     unsigned char* xs = nullptr;  // batched products: x split into bf16 planes
     size_t xs_bytes = 0;
+    unsigned char* hs = nullptr;  // and the down projection's input
+    size_t hs_bytes = 0;
     float* part = nullptr;        // and their K splits' partial sums
     size_t part_bytes = 0;
     unsigned char* kvp = nullptr; // prefill: K and V tiles as bf16 planes
@@ -135,9 +137,9 @@ struct tla_engine {
     long long opt_split = 0;
     int opt_plan = TLA_PLAN_AUTO;
     int opt_group = 0;  // kv heads per aligned-plan workgroup, 0 = per launch
-    int opt_stream_tiles = 0;  // streamed product: token tiles per workgroup, 0 = per shape
-    int opt_split_rows = 0;    // split product: 16-row subtiles per wave, 0 = per shape
-    int opt_split_k = 0;       // split product: K ranges, 0 = per shape
+    int opt_stream_tiles = 0;  // resident product: token tiles per workgroup at most, 0 = per shape
+    int opt_split_rows = 0;    // batched products: 16-row subtiles, 0 = per shape
+    int opt_split_k = 0;       // and K ranges (at least), 0 = per shape
     int n_cu = 256;          // compute units: decode workgroups per launch
 
     bool prof = false;
@@ -404,7 +406,7 @@ int tla_engine_create(const tla_config* cfg, int device, tla_engine** out)
     // Every kernel's code object is loaded now, not at its first launch (a
     // load allocates device memory: tla_decode_noalloc's first call would).
     for (hipError_t (*load)() : {load_decode_code, load_prefill_code, load_gemv_code, load_batch_code,
-                                 load_small_ops_code}) {
+                                 load_product_code, load_small_ops_code}) {
         const hipError_t lerr = load();
         if (lerr != hipSuccess)
             return bail(fail(TLA_ERR_DEVICE, "loading kernel code: %s", hipGetErrorString(lerr)));
@@ -430,6 +432,7 @@ int tla_engine_destroy(tla_engine* e)
     if (e->counters) (void)hipFree(e->counters);
     if (e->fwd) (void)hipFree(e->fwd);
     if (e->xs) (void)hipFree(e->xs);
+    if (e->hs) (void)hipFree(e->hs);
     if (e->part) (void)hipFree(e->part);
     if (e->kvp) (void)hipFree(e->kvp);
     if (e->argmax_slot) (void)hipFree(e->argmax_slot);
@@ -633,6 +636,194 @@ int run_gemv(tla_engine* e, int type, const GemvParams& p)
     GemvParams q = p;
     q.rope = e->rope;  // read by every launch; rotates nothing with rope_rows = 0
     return launch(e, TLA_KERNEL_GEMV, "gemv", [&] { return launch_gemv(type, q, e->stream); });
+}
+
+// Grows a workspace to `bytes` (after the stream's queued work, which may
+// still read it).
+int ensure_buf(tla_engine* e, void** buf, size_t& have, size_t bytes, const char* what)
+{
+    if (bytes <= have) return TLA_OK;
+    TLA_HIP(hipStreamSynchronize(e->stream));
+    if (*buf) TLA_HIP(hipFree(*buf));
+    *buf = nullptr;
+    have = 0;
+    const hipError_t err = hipMalloc(buf, bytes);
+    if (err != hipSuccess)
+        return fail(err == hipErrorOutOfMemory ? TLA_ERR_OUT_OF_MEMORY : TLA_ERR_DEVICE, "%s (%zu bytes): %s",
+                    what, bytes, hipGetErrorString(err));
+    have = bytes;
+    return TLA_OK;
+}
+
+// ---- products of several tokens (split_product.hip) ---------------------------
+
+// Fewest vectors that take the split products; fewer run as matrix-vector
+// launches (which read the weights once per 2 to 8 vectors).  Measured, TinyLlama's
+// matrices: Q4_0 / Q8_0 at 3 vectors 6.9-12.2 us against 7.9-18 us in the
+// matrix-vector launches (and at 2 those give a prompt's first layer the bits
+// of the token path); F16 / F32 at 2; Q6_K, whose decoding costs most, at 8.
+int min_batch(int type) { return type == kQ6_K ? 8 : type == kF16 || type == kF32 ? 2 : 3; }
+
+bool aligned16(const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; }
+
+// Whether n vectors of `cols` columns at x take the split products.
+bool batch_supported(int type, int cols, int n, const float* x, long long x_stride)
+{
+    return n >= min_batch(type) && cols % 64 == 0 && (type != kQ6_K || cols % 256 == 0) && aligned16(x) && x_stride % 4 == 0;
+}
+
+ProductParams product_params(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int cols, int n, int add,
+                             bool pair = false)
+{
+    ProductParams p{};
+    for (int i = 0; i < n_seg; ++i) {
+        p.seg[i] = segs[i];
+        p.total_rows += segs[i].rows;
+    }
+    p.n_seg = n_seg;
+    p.cols = cols;
+    p.row_bytes = weight_row_bytes(type, cols);
+    p.n = n;
+    p.add = add;
+    p.pair = pair ? 1 : 0;
+    plan_product(type, e->n_cu, e->opt_split_rows, e->opt_stream_tiles, e->opt_split_k, &p);
+    return p;
+}
+
+int planes_buf(tla_engine* e, unsigned char** buf, size_t& have, int n, int cols)
+{
+    return ensure_buf(e, reinterpret_cast<void**>(buf), have, product_planes_bytes(n, cols), "split-x workspace");
+}
+
+// The planned product, its input in p.x or p.xs.  deferred (when non-null):
+// the K ranges whose sums are left in e->part for the caller to add
+// (launch_norm_split_rows, launch_reduce_rmsnorm_rows), else 0.
+int run_product(tla_engine* e, int type, ProductParams& p, int* deferred = nullptr)
+{
+    if (deferred) *deferred = 0;
+    if (p.k_splits > 1) {
+        if (int rc = ensure_buf(e, reinterpret_cast<void**>(&e->part), e->part_bytes,
+                                product_part_bytes(p.n, p.total_rows, p.k_splits), "split-product partial sums"))
+            return rc;
+        p.part = e->part;
+        // one segment added to rows of its own width
+        if (deferred && p.n_seg == 1 && p.add && p.seg[0].out_stride == p.total_rows) {
+            p.defer_reduce = 1;
+            *deferred = p.k_splits;
+        }
+    }
+    return launch(e, TLA_KERNEL_GEMV, "product", [&]() -> hipError_t { return launch_product(type, p, e->stream); });
+}
+
+// out_s[t][row] (+)= W_s[row] . x[t] for the n_seg matrices of `segs`, one
+// type, over n tokens (x rows x_stride floats apart): split products where
+// batch_supported, else matrix-vector launches.
+int matrix_batch(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int cols, const float* x,
+                 long long x_stride, int n, int add, int* deferred = nullptr)
+{
+    if (deferred) *deferred = 0;
+    if (batch_supported(type, cols, n, x, x_stride)) {
+        ProductParams p = product_params(e, type, segs, n_seg, cols, n, add);
+        p.x = x;
+        p.x_stride = x_stride;
+        if (p.kind != kProductDirect) {
+            if (int rc = planes_buf(e, &e->xs, e->xs_bytes, n, cols)) return rc;
+            p.planes = 1;
+            p.xs = e->xs;
+            if (int rc = launch(e, TLA_KERNEL_GEMV, "split rows", [&]() -> hipError_t {
+                    return launch_split_rows(x, x_stride, n, cols, false, e->xs, e->stream);
+                }))
+                return rc;
+        }
+        return run_product(e, type, p, deferred);
+    }
+    const int chunk = gemv_chunk(n, cols);
+    for (int t0 = 0; t0 < n; t0 += chunk) {
+        GemvParams p{};
+        for (int i = 0; i < n_seg; ++i) {
+            p.seg[i] = segs[i];
+            p.seg[i].out = segs[i].out + static_cast<long long>(t0) * segs[i].out_stride;
+            p.total_rows += segs[i].rows;
+        }
+        p.n_seg = n_seg;
+        p.cols = cols;
+        p.row_bytes = static_cast<int>(weight_row_bytes(type, cols));
+        p.n_vec = std::min(chunk, n - t0);
+        p.x = x + static_cast<long long>(t0) * x_stride;
+        p.x_stride = x_stride;
+        p.add = add;
+        if (int rc = run_gemv(e, type, p)) return rc;
+    }
+    return TLA_OK;
+}
+
+// The same over rmsnorm(x[t], norm_w, eps), for dense rows x that
+// batch_supported takes (norm_w 16-byte aligned): the norm inside a direct
+// product, else in the launch that writes the planes.  pending (K ranges left
+// in e->part by the product before): those sums are added to x first, by
+// that launch.  With pair (two segments, gate and up), e->hs receives the
+// planes of silu(gate) * up; the segments' outs may then be NULL if
+// paired_product says so.
+int norm_product(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int cols, float* x, const float* norm_w,
+                 float eps, int n, int pending, bool pair)
+{
+    ProductParams p = product_params(e, type, segs, n_seg, cols, n, 0, pair);
+    if (pair) {
+        if (int rc = planes_buf(e, &e->hs, e->hs_bytes, n, segs[0].rows)) return rc;
+        p.hs = e->hs;
+    }
+    if (p.kind == kProductDirect && !pending && cols <= kProductMaxNorm) {
+        p.x = x;
+        p.x_stride = cols;
+        p.norm_w = norm_w;
+        p.eps = eps;
+        return run_product(e, type, p);
+    }
+    if (int rc = planes_buf(e, &e->xs, e->xs_bytes, n, cols)) return rc;
+    if (int rc = launch(e, TLA_KERNEL_GEMV, "norm + split rows", [&]() -> hipError_t {
+            return launch_norm_split_rows(x, e->part, pending, n, cols, norm_w, eps, e->xs, e->stream);
+        }))
+        return rc;
+    p.planes = 1;
+    p.xs = e->xs;
+    return run_product(e, type, p);
+}
+
+// Whether the gate and up product of this shape runs paired (its epilogue
+// writes the planes of silu(gate) * up): where the unpaired one would not
+// take the tiled kernel, and rows are whole blocks.
+bool paired_product(tla_engine* e, int type, int n_ff, int cols, int n)
+{
+    const GemvSegment segs[2] = {{nullptr, nullptr, n_ff, 0}, {nullptr, nullptr, n_ff, 0}};
+    return n_ff % 64 == 0 && product_params(e, type, segs, 2, cols, n, 0).kind != kProductTiled &&
+           product_params(e, type, segs, 2, cols, n, 0, true).k_splits == 1;
+}
+
+// x[t] += W_down . (silu(gate_t) * up_t) for n token rows, gate and up from
+// rmsnorm(x[t]) (src/forward.cpp:215-228), for rows that batch_supported
+// takes: hb [n][2][n_ff] receives the raw gate and up projections when keep_hb (it may
+// otherwise be left unwritten).
+int ffn_batch(tla_engine* e, int type, float* x, const float* norm_w, float eps, const void* w_gate, const void* w_up,
+              const void* w_down, int n_ff, int embd, int n, float* hb, bool keep_hb, int pending, int* deferred)
+{
+    const auto U = [](const void* w) { return static_cast<const unsigned char*>(w); };
+    const bool pair = paired_product(e, type, n_ff, embd, n);
+    const bool raw = keep_hb || !pair;
+    const GemvSegment gu[2] = {{U(w_gate), raw ? hb : nullptr, n_ff, 2LL * n_ff},
+                               {U(w_up), raw ? hb + n_ff : nullptr, n_ff, 2LL * n_ff}};
+    if (int rc = norm_product(e, type, gu, 2, embd, x, norm_w, eps, n, pending, pair)) return rc;
+    if (!pair) {
+        if (int rc = planes_buf(e, &e->hs, e->hs_bytes, n, n_ff)) return rc;
+        if (int rc = launch(e, TLA_KERNEL_GEMV, "swiglu rows", [&]() -> hipError_t {
+                return launch_split_rows(hb, 2LL * n_ff, n, n_ff, true, e->hs, e->stream);
+            }))
+            return rc;
+    }
+    const GemvSegment down{U(w_down), x, embd, embd};
+    ProductParams p = product_params(e, type, &down, 1, n_ff, n, 1);
+    p.planes = 1;
+    p.xs = e->hs;
+    return run_product(e, type, p, deferred);
 }
 
 }  // namespace
@@ -956,27 +1147,6 @@ int tla_rope_attention_host(tla_engine* e, float* out_host, const float* qkv_hos
     return ok();
 }
 
-namespace {
-
-// Grows a workspace to `bytes` (after the stream's queued work, which may
-// still read it).
-int ensure_buf(tla_engine* e, void** buf, size_t& have, size_t bytes, const char* what)
-{
-    if (bytes <= have) return TLA_OK;
-    TLA_HIP(hipStreamSynchronize(e->stream));
-    if (*buf) TLA_HIP(hipFree(*buf));
-    *buf = nullptr;
-    have = 0;
-    const hipError_t err = hipMalloc(buf, bytes);
-    if (err != hipSuccess)
-        return fail(err == hipErrorOutOfMemory ? TLA_ERR_OUT_OF_MEMORY : TLA_ERR_DEVICE, "%s (%zu bytes): %s",
-                    what, bytes, hipGetErrorString(err));
-    have = bytes;
-    return TLA_OK;
-}
-
-}  // namespace
-
 int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layers, int flags,
                 float* out_dev, const float* q_dev, const float* k_dev, const float* v_dev,
                 float* key_cache_dev, float* value_cache_dev)
@@ -1065,8 +1235,6 @@ int gemv1(tla_engine* e, int type, const void* w, float* out, int rows, int cols
     p.add = add;
     return run_gemv(e, type, p);
 }
-
-bool aligned16(const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; }
 
 // Shapes, types and pointers of a model against the engine's config.
 int check_model(const tla_engine* e, const tla_model* m)
@@ -1291,177 +1459,12 @@ int forward_step(tla_engine* e, const tla_model* m, const FwdBufs& b, float* kc,
     return TLA_OK;
 }
 
-// out[t][rows] = W . x[t] for n vectors x [n][cols], in launches of up to
-// gemv_chunk vectors.
-int gemv_rows(tla_engine* e, int type, const void* w, float* out, int rows, int cols, const float* x, int n)
-{
-    const int chunk = gemv_chunk(n, cols);
-    for (int t0 = 0; t0 < n; t0 += chunk) {
-        GemvParams p{};
-        p.seg[0] = {static_cast<const unsigned char*>(w), out + static_cast<long long>(t0) * rows, rows, rows};
-        p.n_seg = 1;
-        p.total_rows = rows;
-        p.cols = cols;
-        p.row_bytes = static_cast<int>(weight_row_bytes(type, cols));
-        p.n_vec = std::min(chunk, n - t0);
-        p.x = x + static_cast<long long>(t0) * cols;
-        p.x_stride = cols;
-        if (int rc = run_gemv(e, type, p)) return rc;
-    }
-    return TLA_OK;
-}
-
-// Token batches at least this long (and past the streamed product's range)
-// take the split product below; shorter ones the multi-vector GEMV (weights
-// read once per group of up to 8 tokens).
-constexpr int kBatchMinTokens = 16;
-
-// out_s[t][row] (+)= W_s[row] . x[t] as the split product (split_product.hip):
-// x split into three bf16 planes, then one launch over all segments, the
-// weights dequantised in registers.  Two 16-row subtiles per wave where
-// that still gives half the CUs a workgroup, else one; then K cut into
-// ranges of at least 8 blocks until the grid holds about 2.5 workgroups per
-// CU (each a workgroup walking its range, the ranges' sums added in order
-// by a second launch).  A workgroup's blocks follow one another at about a
-// memory round trip each, so shorter ranges and more resident workgroups
-// are what shortens a product.  Same box, TinyLlama's four matrices, Q4_0,
-// rows per wave x K ranges swept: at 512 tokens gate | up 129 us (2 x 1)
-// against 174 us with 4 rows per wave, W_down 73 us (2 x 4-6) against 107
-// (1 x 2); at 128 tokens every matrix within 2 us of its best.
-int split_batch(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int total, int cols, const float* x,
-                long long x_stride, int n, int add, int* deferred = nullptr)
-{
-    if (deferred) *deferred = 0;
-    if (int rc = ensure_buf(e, reinterpret_cast<void**>(&e->xs), e->xs_bytes, split_x_bytes(n, cols), "split-x workspace")) return rc;
-    SplitParams p{};
-    for (int i = 0; i < n_seg; ++i) p.seg[i] = segs[i];
-    p.n_seg = n_seg;
-    p.total_rows = total;
-    p.cols = cols;
-    p.row_bytes = weight_row_bytes(type, cols);
-    p.xs = e->xs;
-    p.n = n;
-    p.n_sub = split_tokens(n) / 16;
-    p.add = add;
-    const long long token_tiles = p.n_sub / 4;
-    auto groups = [&](int rw) { return (total + 64LL * rw - 1) / (64LL * rw) * token_tiles; };
-    p.rows_per_wave = 2 * groups(2) >= e->n_cu ? 2 : 1;
-    if (e->opt_split_rows > 0) p.rows_per_wave = e->opt_split_rows;
-    const int n_blk = cols / 32;
-    const long long g = groups(p.rows_per_wave), target = 5LL * e->n_cu / 2;
-    int splits = static_cast<int>(std::min<long long>((target + g - 1) / g, n_blk / 8));
-    if (e->opt_split_k > 0) splits = e->opt_split_k;
-    splits = std::max(1, std::min(splits, n_blk));
-    p.blk_per_split = (n_blk + splits - 1) / splits;
-    p.k_splits = (n_blk + p.blk_per_split - 1) / p.blk_per_split;
-    if (p.k_splits > 1) {
-        if (int rc = ensure_buf(e, reinterpret_cast<void**>(&e->part), e->part_bytes, split_part_bytes(n, total, p.k_splits),
-                                "split-product partial sums"))
-            return rc;
-        p.part = e->part;
-        // one segment added to rows of its own width: the caller may add the
-        // ranges' sums itself, with the rmsnorm that follows
-        // (launch_reduce_rmsnorm_rows), instead of a launch of their own
-        if (deferred && n_seg == 1 && add && segs[0].out_stride == total) {
-            p.defer_reduce = 1;
-            *deferred = p.k_splits;
-        }
-    }
-    if (int rc = launch(e, TLA_KERNEL_GEMV, "split rows",
-                        [&]() -> hipError_t { return launch_split_rows(x, x_stride, n, cols, e->xs, e->stream); }))
-        return rc;
-    return launch(e, TLA_KERNEL_GEMV, "split product",
-                  [&]() -> hipError_t { return launch_split_product(type, p, e->stream); });
-}
-
-// out_s[t][row] (+)= W_s[row] . x[t] for the n_seg matrices of `segs`, one
-// type, over n tokens (x rows x_stride floats apart).
-// Batches of stream_min_tokens(type) .. kStreamMaxTokens vectors multiply F32
-// / F16 / Q8_0 / Q4_0 weights where they lie, dequantised in registers by
-// stream_product_kernel; a library product on an fp32 copy of the weights
-// ran far below the MFMA rate at these widths (Q4_0 prompts of 33 / 48 / 64
-// tokens 2.79 / 3.22 / 3.60 ms streamed against 3.60 / 3.64 / 3.65 ms), and
-// the
-// multi-vector GEMVs read the weights once per 2-6 vectors (Q4_0 prompts of
-// 3 / 8 / 15 tokens 1.67 / 1.82 / ~2.0 ms streamed against 1.89 / 4.21 /
-// 7.25 ms).  At 2 tokens the GEMVs keep the quantised formats (Q4_0 1.53
-// against 1.63 ms, Q8_0 1.59 against 1.62) but not F16 / F32 (1.69 / 1.93
-// against 1.41 / 1.72 ms).  Past 64 vectors the split product takes over:
-// each 16-row workgroup of the streamed product loads all of x itself.
-constexpr int kStreamMaxTokens = 64;
-
-int stream_min_tokens(int type) { return type == kF16 || type == kF32 ? 2 : 3; }
-
-bool use_stream(int type, int cols, int n, long long x_stride)
-{
-    return stream_supported(type) && n >= stream_min_tokens(type) && n <= kStreamMaxTokens && cols % 32 == 0 &&
-           x_stride % 4 == 0;
-}
-
-int stream_batch(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int total, int cols,
-                 const float* x, long long x_stride, int n, int add)
-{
-    StreamParams p{};
-    for (int i = 0; i < n_seg; ++i) p.seg[i] = segs[i];
-    p.n_seg = n_seg;
-    p.total_rows = total;
-    p.cols = cols;
-    p.row_bytes = weight_row_bytes(type, cols);
-    p.x = x;
-    p.x_stride = x_stride;
-    p.n = n;
-    p.add = add;
-    // token tiles of 16 per workgroup: one for matrices of at most 128 row
-    // tiles (their workgroups are too few to fill the CUs otherwise; W_o and
-    // W_down at TinyLlama's shapes, 32 tokens: 11.6 against 15.2 us and 22.4
-    // against 30.1 us), else as many as kStreamMaxTiles allows (W_qkv,
-    // gate + up: 15.4 against 19.7 us, 40.6 against 52.7 us)
-    const int nt = (n + 15) / 16;
-    p.tiles = e->opt_stream_tiles > 0 ? e->opt_stream_tiles
-              : (total + 15) / 16 <= 128 ? 1
-                                         : std::min(nt, kStreamMaxTiles);
-    return launch(e, TLA_KERNEL_GEMV, "streamed product",
-                  [&]() -> hipError_t { return launch_stream_product(type, p, e->stream); });
-}
-
-// deferred (when non-null): the K ranges whose sums a split product left in
-// e->part for the caller to add (launch_reduce_rmsnorm_rows), else 0.
-int matrix_batch(tla_engine* e, int type, const GemvSegment* segs, int n_seg, int cols, const float* x,
-                 long long x_stride, int n, int add, int* deferred = nullptr)
-{
-    if (deferred) *deferred = 0;
-    int total = 0;
-    for (int i = 0; i < n_seg; ++i) total += segs[i].rows;
-    if (use_stream(type, cols, n, x_stride)) return stream_batch(e, type, segs, n_seg, total, cols, x, x_stride, n, add);
-    if (n >= kBatchMinTokens && cols % 32 == 0 && (type != kQ6_K || cols % 256 == 0) && x_stride % 4 == 0 &&
-        reinterpret_cast<std::uintptr_t>(x) % 16 == 0)
-        return split_batch(e, type, segs, n_seg, total, cols, x, x_stride, n, add, deferred);
-    const int chunk = std::max(1, std::min({n, kGemvMaxVec, kGemvLdsBytes / gemv_lds_per_vec(cols)}));
-    for (int t0 = 0; t0 < n; t0 += chunk) {
-        GemvParams p{};
-        for (int i = 0; i < n_seg; ++i) {
-            p.seg[i] = segs[i];
-            p.seg[i].out = segs[i].out + static_cast<long long>(t0) * segs[i].out_stride;
-        }
-        p.n_seg = n_seg;
-        p.total_rows = total;
-        p.cols = cols;
-        p.row_bytes = static_cast<int>(weight_row_bytes(type, cols));
-        p.n_vec = std::min(chunk, n - t0);
-        p.x = x + static_cast<long long>(t0) * x_stride;
-        p.x_stride = x_stride;
-        p.add = add;
-        if (int rc = run_gemv(e, type, p)) return rc;
-    }
-    return TLA_OK;
-}
-
 // The prompt as one batch (n_tok tokens at positions pos0..): embeddings,
 // then per layer rmsnorm + Q/K/V over all tokens, the causal prefill
 // attention (RoPE + append in-kernel), W_o + residual and the FFN;
-// logits of the last token only (when `logits` is non-null).  Every
-// product is a matrix_batch: multi-vector GEMVs, streamed products or
-// split products by the prompt's length.
+// logits of the last token only (when `logits` is non-null).  The products
+// are split products (norm_product, ffn_batch, matrix_batch), or matrix-vector
+// launches for one or two tokens.
 int prompt_step(tla_engine* e, const tla_model* m, const FwdBufs& b, float* kc, float* vc,
                 const int* tokens_dev, int n_tok, int pos0, float* logits)
 {
@@ -1474,9 +1477,9 @@ int prompt_step(tla_engine* e, const tla_model* m, const FwdBufs& b, float* kc, 
     const auto U = [](const void* w) { return static_cast<const unsigned char*>(w); };
     const int n_layers = e->cfg.n_layers;
     // The W_o and W_down products add to x; where their K ranges' sums are
-    // left in e->part (pending), the rmsnorm rows launch after them adds
-    // them first (one launch for both), before any other product reuses
-    // e->part.  After the last layer x is added to by the product itself.
+    // left in e->part (pending), the norm launch after them adds them first
+    // (one launch for both), before any other product reuses e->part.  After
+    // the last layer x is added to by the product itself.
     int pending = 0;
     auto norm_rows = [&](const float* w) -> int {
         const hipError_t err = pending ? launch_reduce_rmsnorm_rows(b.x, e->part, pending, b.xb, w, n_tok, embd,
@@ -1485,22 +1488,26 @@ int prompt_step(tla_engine* e, const tla_model* m, const FwdBufs& b, float* kc, 
         pending = 0;
         return check_hip(err, "rmsnorm rows");
     };
+    const auto batch = [&](int type, const float* norm_w) {
+        return batch_supported(type, embd, n_tok, b.x, embd) && aligned16(norm_w);
+    };
     for (int l = 0; l < n_layers; ++l) {
         const tla_layer_weights& L = m->layers[l];
-        auto product = [&](int type, const GemvSegment* segs, int n_seg, int cols, const float* x,
-                           long long x_stride, int add) -> int {
-            return matrix_batch(e, type, segs, n_seg, cols, x, x_stride, n_tok, add);
-        };
-        // rmsnorm rows, then Q/K/V (src/forward.cpp:180-190)
-        if (int rc = norm_rows(L.attn_norm)) return rc;
-        if (L.type_q == L.type_k && L.type_q == L.type_v) {
-            const GemvSegment segs[3] = {{U(L.wq), b.q, embd, embd}, {U(L.wk), b.k, kv, kv}, {U(L.wv), b.v, kv, kv}};
-            if (int rc = product(L.type_q, segs, 3, embd, b.xb, embd, 0)) return rc;
+        // rmsnorm, then Q/K/V (src/forward.cpp:180-190)
+        const GemvSegment qkv[3] = {{U(L.wq), b.q, embd, embd}, {U(L.wk), b.k, kv, kv}, {U(L.wv), b.v, kv, kv}};
+        const bool same = L.type_q == L.type_k && L.type_q == L.type_v;
+        if (same && batch(L.type_q, L.attn_norm)) {
+            if (int rc = norm_product(e, L.type_q, qkv, 3, embd, b.x, L.attn_norm, eps, n_tok, pending, false)) return rc;
+            pending = 0;
         } else {
-            const GemvSegment sq{U(L.wq), b.q, embd, embd}, sk{U(L.wk), b.k, kv, kv}, sv{U(L.wv), b.v, kv, kv};
-            if (int rc = matrix_batch(e, L.type_q, &sq, 1, embd, b.xb, embd, n_tok, 0)) return rc;
-            if (int rc = matrix_batch(e, L.type_k, &sk, 1, embd, b.xb, embd, n_tok, 0)) return rc;
-            if (int rc = matrix_batch(e, L.type_v, &sv, 1, embd, b.xb, embd, n_tok, 0)) return rc;
+            if (int rc = norm_rows(L.attn_norm)) return rc;
+            if (same) {
+                if (int rc = matrix_batch(e, L.type_q, qkv, 3, embd, b.xb, embd, n_tok, 0)) return rc;
+            } else {
+                if (int rc = matrix_batch(e, L.type_q, &qkv[0], 1, embd, b.xb, embd, n_tok, 0)) return rc;
+                if (int rc = matrix_batch(e, L.type_k, &qkv[1], 1, embd, b.xb, embd, n_tok, 0)) return rc;
+                if (int rc = matrix_batch(e, L.type_v, &qkv[2], 1, embd, b.xb, embd, n_tok, 0)) return rc;
+            }
         }
         // RoPE + append + causal attention (src/forward.cpp:192-208)
         if (int rc = tla_prefill(e, pos0, n_tok, l, 1, TLA_ROTATE, b.att, b.q, b.k, b.v, kc, vc)) return rc;
@@ -1509,19 +1516,23 @@ int prompt_step(tla_engine* e, const tla_model* m, const FwdBufs& b, float* kc, 
             const GemvSegment so{U(L.wo), b.x, embd, embd};
             if (int rc = matrix_batch(e, L.type_o, &so, 1, embd, b.att, embd, n_tok, 1, &pending)) return rc;
         }
-        // FFN (src/forward.cpp:215-228): rmsnorm rows, gate and up into
-        // hb [t][gate | up], SiLU x up in place, x += W_down . h
-        if (int rc = norm_rows(L.ffn_norm)) return rc;
-        {
-            const GemvSegment segs[2] = {{U(L.w_gate), b.hb, ff, 2LL * ff}, {U(L.w_up), b.hb + ff, ff, 2LL * ff}};
-            if (int rc = product(L.type_ffn, segs, 2, embd, b.xb, embd, 0)) return rc;
-        }
-        if (int rc = check_hip(launch_swiglu_rows(b.hb, n_tok, ff, e->stream), "swiglu rows")) return rc;
-        {
-            const GemvSegment sd{U(L.w_down), b.x, embd, embd};
-            if (int rc = matrix_batch(e, L.type_ffn, &sd, 1, ff, b.hb, 2LL * ff, n_tok, 1,
-                                      l + 1 < n_layers ? &pending : nullptr))
+        // FFN (src/forward.cpp:215-228)
+        int* const defer = l + 1 < n_layers ? &pending : nullptr;
+        if (batch(L.type_ffn, L.ffn_norm) && (L.type_ffn != kQ6_K || ff % 256 == 0)) {
+            const int before = pending;
+            pending = 0;
+            if (int rc = ffn_batch(e, L.type_ffn, b.x, L.ffn_norm, eps, L.w_gate, L.w_up, L.w_down, ff, embd, n_tok,
+                                   b.hb, false, before, defer))
                 return rc;
+        } else {
+            // rmsnorm rows, gate and up into hb [t][gate | up], SiLU x up in
+            // place, x += W_down . h
+            if (int rc = norm_rows(L.ffn_norm)) return rc;
+            const GemvSegment gu[2] = {{U(L.w_gate), b.hb, ff, 2LL * ff}, {U(L.w_up), b.hb + ff, ff, 2LL * ff}};
+            if (int rc = matrix_batch(e, L.type_ffn, gu, 2, embd, b.xb, embd, n_tok, 0)) return rc;
+            if (int rc = check_hip(launch_swiglu_rows(b.hb, n_tok, ff, e->stream), "swiglu rows")) return rc;
+            const GemvSegment sd{U(L.w_down), b.x, embd, embd};
+            if (int rc = matrix_batch(e, L.type_ffn, &sd, 1, ff, b.hb, 2LL * ff, n_tok, 1, defer)) return rc;
         }
     }
     if (logits)
@@ -1936,8 +1947,8 @@ int tla_set_option(tla_engine* e, int option, long long value)
         e->opt_group = static_cast<int>(value);
         return ok();
     case TLA_OPT_STREAM_TILES:
-        if (value < 0 || value > kStreamMaxTiles)
-            return fail(TLA_ERR_INVALID_ARGUMENT, "stream tiles %lld not in [0, %d]", value, kStreamMaxTiles);
+        if (value < 0 || value > 4)
+            return fail(TLA_ERR_INVALID_ARGUMENT, "stream tiles %lld not in [0, 4]", value);
         e->opt_stream_tiles = static_cast<int>(value);
         return ok();
     case TLA_OPT_SPLIT_ROWS:

@@ -1,5 +1,5 @@
-// split_product_kernel: the projections of a prompt of many tokens
-// (tla_matmul_batch, tla_prefill_forward) as bf16 matrix-core products that
+// Split products: the projections of several tokens (tla_matmul_batch,
+// tla_prefill_forward, a layer over several sequences) as bf16 matrix-core products that
 // keep fp32 accuracy: the batched form of the matmuls forward() makes per
 // token (src/forward.cpp:180-228, matmul() src/ops.cpp:959-983; weight
 // blocks src/gguf.h:56-135).
@@ -23,41 +23,56 @@
 // times their fp32 rate, so 3-6 bf16 products per fp32 multiply-add still
 // leave the product well inside it.
 //
-// Layout.  split_rows_kernel writes x once per product as bf16 planes in
-// the order the A operand reads them: for each 32-column block kb, plane p
-// and 16-token subtile s, 1 KiB whose 16-byte piece 16 g + i holds plane p
-// of x[16 s + i][32 kb + 8 g .. + 7] (tokens past n are zeros).  A wave's
-// operand read is then 1 KiB contiguous, from global memory into LDS and
-// from LDS into registers, without bank conflicts.
+// Layout.  x as bf16 planes, in the order the A operand reads them: for each
+// tile of 16 tokens, 32-column block kb and plane, 1 KiB whose 16-byte piece
+// 16 g + i holds the plane of x[16 tile + i][32 kb + 8 g .. + 7].  A wave's
+// operand read is then 1 KiB contiguous, and a wave's K slice of a tile one
+// run of memory.  Rows past the last token are never used: a row of A only
+// reaches the same row of the result.
 //
-// Tiling.  A workgroup of 4 waves owns 64 kRW weight rows x 64 tokens (4
-// token subtiles); wave w owns rows 16 kRW w .. + 16 kRW - 1 for all 64
-// tokens, so each x plane read from LDS feeds kRW products.  The tokens are
-// the A operand and the weight rows the B operand of
+// The tokens are the A operand and the weight rows the B operand of
 // v_mfma_f32_16x16x32_bf16: lane l = 16 g + j supplies token j's and row j's
 // values for columns 8 g .. 8 g + 7 of the block, and holds the sums of
-// tokens 4 g .. 4 g + 3 for row j -- one block scale per lane.  The x
-// blocks pass through a ring of three LDS stages (12 KiB each: three planes
-// of 64 tokens), staged through registers two blocks ahead; each wave loads
-// its rows' weights three blocks ahead and dequantises them in registers.
-// Every output is one wave's sum in a fixed order: the same bits on every
-// run and for any grid.
+// tokens 4 g .. 4 g + 3 for row j -- one block scale per lane.  The weights
+// are dequantised in registers.
+//
+// Three kernels, by the number of tokens (plan_product):
+//   direct    up to 16 tokens, or few rows: K over the waves of a workgroup,
+//             x split (and normalised) by the workgroup itself;
+//   resident  more tokens: a workgroup keeps its rows' decoded weights in
+//             registers and streams the x planes of all token tiles past them;
+//   tiled     past 192 tokens for the shapes whose decoded weights are too
+//             many for the registers: a 64 kRW row x 64 token tile per
+//             workgroup, x through LDS.
+// Every output is a sum in a fixed order: the same bits on every run and for
+// any grid.
+#include <algorithm>
+#include <type_traits>
+
 #include "batch.h"
 #include "bf16_split.h"
+#include "row_math.h"
 
 namespace tla {
 namespace {
 
-constexpr int kThreads = 256;  // 4 waves
-constexpr int kWaves = kThreads / 64;
-constexpr int kTW = 4;         // token subtiles of 16 per workgroup
-constexpr int kRing = 3;       // LDS stages, x register stages and weight register stages
-constexpr int kStageBytes = 3 * kTW * 1024;
-constexpr int kChunksPerWave = kStageBytes / 1024 / kWaves;  // 1 KiB copies per wave and stage
-static_assert(kChunksPerWave * 1024 * kWaves == kStageBytes, "a stage is whole chunks per wave");
+constexpr int kThreads = 256;          // the row kernels, range sums
+constexpr int kWaves = 8;              // waves per direct / resident workgroup
+constexpr int kMaxSlice = 8;           // resident: 32-column blocks per wave, at most
+constexpr int kRangeBlocks = kWaves * kMaxSlice;  // and so blocks of one K range, at most
+constexpr int kRing = 4;               // resident: blocks of x ahead per wave
+constexpr int kMaxRows = 3;            // 16-row subtiles per workgroup, at most
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef __attribute__((address_space(1))) void* global_ptr;
+
+// the tiled product
+constexpr int kTileThreads = 256;
+constexpr int kTileWaves = kTileThreads / 64;
+constexpr int kTW = 4;                 // token tiles per workgroup
+constexpr int kStages = 3;             // LDS stages, x register stages and weight register stages
+constexpr int kStageBytes = 3 * kTW * 1024;
+constexpr int kChunksPerWave = kStageBytes / 1024 / kTileWaves;  // 1 KiB copies per wave and stage
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -73,43 +88,147 @@ __device__ __forceinline__ float half_to_float(unsigned h)
     return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(h)));
 }
 
-// Byte offset of plane p of block kb, token subtile s, in the split x.
-__device__ __forceinline__ long long plane_chunk(int kb, int p, int s, int n_sub)
+// silu(v) * u, with the reference's operation order (src/ops.cpp:1107-1148).
+__device__ __forceinline__ float gated(float v, float u)
 {
-    return (static_cast<long long>(kb * 3 + p) * n_sub + s) * 1024;
+    const float sigmoid = 1.0f / (1.0f + expf(-v));
+    return (v * sigmoid) * u;
 }
 
-// One thread per (block kb, token subtile s, lane slot 16 g + i): the three
-// planes of x[16 s + i][32 kb + 8 g .. + 7].
-__global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __restrict__ x, long long x_stride,
-                                                              int n, int n_sub, int n_blk,
-                                                              unsigned char* __restrict__ xs)
+// Byte offset of plane p of block kb, token tile s, in the split x.
+__device__ __forceinline__ long long plane_chunk(int s, int kb, int p, int n_blk)
 {
-    const long long id = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
-    if (id >= static_cast<long long>(n_blk) * n_sub * 64) return;
-    const int slot = static_cast<int>(id & 63), g = slot >> 4, i = slot & 15;
-    const long long rest = id >> 6;
-    const int s = static_cast<int>(rest % n_sub), kb = static_cast<int>(rest / n_sub);
-    const int t = 16 * s + i;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (t < n) {
-        const float4* src = reinterpret_cast<const float4*>(x + t * x_stride + 32 * kb + 8 * g);
-        const float4 a = src[0], b = src[1];
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    }
-    bf16x8 p0, p1, p2;
+    return (static_cast<long long>(s * n_blk + kb) * 3 + p) * 1024;
+}
+
+// The three planes of eight values.  An infinity keeps its products: (inf, 0,
+// 0), not (inf, NaN, NaN); a finite value that rounds to a bf16 infinity is
+// truncated instead (its rest still fits the other two pieces).
+__device__ __forceinline__ void split_any(const float (&v)[8], bf16x8 (&x)[3])
+{
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         __bf16 a, b, c;
         split3(v[e], a, b, c);
-        p0[e] = a;
-        p1[e] = b;
-        p2[e] = c;
+        if (__builtin_isinf(static_cast<float>(a))) {
+            if (__builtin_isinf(v[e])) {
+                b = c = static_cast<__bf16>(0.f);
+            } else {
+                const float t = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v[e]) & 0xFFFF0000u);
+                a = static_cast<__bf16>(t);
+                split2(v[e] - t, b, c);
+            }
+        }
+        x[0][e] = a;
+        x[1][e] = b;
+        x[2][e] = c;
     }
-    *reinterpret_cast<bf16x8*>(xs + plane_chunk(kb, 0, s, n_sub) + 16 * slot) = p0;
-    *reinterpret_cast<bf16x8*>(xs + plane_chunk(kb, 1, s, n_sub) + 16 * slot) = p1;
-    *reinterpret_cast<bf16x8*>(xs + plane_chunk(kb, 2, s, n_sub) + 16 * slot) = p2;
+}
+
+// Eight values of token t, columns 8 c8 .. + 7, into the planes.
+__device__ __forceinline__ void store_pieces(unsigned char* xs, int t, int c8, int n_blk, const float (&v)[8])
+{
+    bf16x8 x[3];
+    split_any(v, x);
+    const int slot = 16 * (c8 & 3) + (t & 15);
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl)
+        *reinterpret_cast<bf16x8*>(xs + plane_chunk(t >> 4, c8 >> 2, pl, n_blk) + 16 * slot) = x[pl];
+}
+
+__device__ __forceinline__ void load8(const float* p, float (&v)[8])
+{
+    const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+}
+
+// One thread per (token tile s, block kb, lane slot 16 g + i): the three
+// planes of x[16 s + i][32 kb + 8 g .. + 7].
+// kGated: x rows are [gate | up] (2 cols floats) and the value is silu(gate)
+// * up, with the reference's operation order (src/ops.cpp:1107-1148).
+template <bool kGated>
+__global__ __launch_bounds__(kThreads) void split_rows_kernel(const float* __restrict__ x, long long x_stride,
+                                                              int n, int n_tiles, int n_blk,
+                                                              unsigned char* __restrict__ xs)
+{
+    const long long id = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
+    if (id >= static_cast<long long>(n_blk) * n_tiles * 64) return;
+    const int slot = static_cast<int>(id & 63), g = slot >> 4, i = slot & 15;
+    const long long rest = id >> 6;
+    const int kb = static_cast<int>(rest % n_blk), t = 16 * static_cast<int>(rest / n_blk) + i;
+    if (t >= n) return;
+    float v[8];
+    const float* const row = x + t * x_stride + 32 * kb + 8 * g;
+    load8(row, v);
+    if constexpr (kGated) {
+        float u[8];
+        load8(row + 32 * n_blk, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = gated(v[e], u[e]);
+    }
+    store_pieces(xs, t, 4 * kb + g, n_blk, v);
+}
+
+// rmsnorm of each row of x into the planes, one workgroup per row (its pieces
+// are 16-byte stores into 16-token chunks; one launch of ~5 us at 64 rows in place of
+// the norm's and the split's).  With
+// k_splits > 0 the row first takes the K-range sums part[z][t][c] of the
+// product before (in range order, as range_sum_kernel adds them), and is
+// written back.
+__global__ __launch_bounds__(kThreads) void norm_split_rows_kernel(float* x, const float* part, int k_splits,
+                                                                   long long plane, const float* w, int cols,
+                                                                   float eps, unsigned char* xs)
+{
+    __shared__ float s_sum[kThreads / 64];
+    const int t = blockIdx.x;
+    float* const row = x + static_cast<long long>(t) * cols;
+    const float* const prow = part + static_cast<long long>(t) * cols;
+    const auto take = [&](int c8, float (&v)[8]) __attribute__((always_inline)) {
+        load8(row + 8 * c8, v);
+        if (k_splits > 0) {
+            float a[8];
+            load8(prow + 8 * c8, a);
+            for (int z = 1; z < k_splits; ++z) {
+                float b[8];
+                load8(prow + z * plane + 8 * c8, b);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[e] += b[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += a[e];
+        }
+    };
+    float first[8];
+    float ss = 0.f;
+    for (int c8 = threadIdx.x; c8 < cols / 8; c8 += kThreads) {
+        float v[8];
+        take(c8, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
+        if (k_splits > 0) {
+            reinterpret_cast<float4*>(row + 8 * c8)[0] = make_float4(v[0], v[1], v[2], v[3]);
+            reinterpret_cast<float4*>(row + 8 * c8)[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+        if (c8 == static_cast<int>(threadIdx.x))
+#pragma unroll
+            for (int e = 0; e < 8; ++e) first[e] = v[e];
+    }
+    ss = block_sum<kThreads>(ss, s_sum);
+    const float rms = 1.0f / sqrtf(ss / static_cast<float>(cols) + eps);
+    for (int c8 = threadIdx.x; c8 < cols / 8; c8 += kThreads) {
+        float v[8], nw[8];
+        load8(w + 8 * c8, nw);
+        if (c8 == static_cast<int>(threadIdx.x)) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = first[e];
+        } else {
+            load8(row + 8 * c8, v);  // this thread's own stores, read back
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = v[e] * rms * nw[e];
+        store_pieces(xs, t, c8, cols / 32, v);
+    }
 }
 
 // One lane's raw weight bits for one row and block, as loaded (decoded only
@@ -147,7 +266,8 @@ struct Fmt {
 
 // Loads of block kb of one weight row (wrow) for lane group g.  kRowLoads:
 // the memory instructions they are at least (separate addresses the
-// compiler cannot merge), which the kernel's wait for its LDS copies counts.
+// compiler cannot merge), which the tiled kernel's wait for its LDS copies
+// counts.
 template <int kType>
 constexpr int kRowLoads = kType == kF32 ? 2 : kType == kQ6_K ? 4 : 1;
 
@@ -175,16 +295,18 @@ __device__ __forceinline__ void load_w(WRaw<kType>& w, const unsigned char* wrow
         __builtin_memcpy(&d, sb + 208, 2);
         w.sd = sc | (static_cast<unsigned>(d) << 16);
     } else {
-        // One 12-byte load: lanes of g = 0 (Q4_0: g = 0 and 2) read bytes
-        // 0..11 of the block (the scale, then their 8 bytes at 2..9); the
-        // others read the 12 bytes ending with their 8 (at 4..11) and take
-        // the scale from their row's lane of g = 0.  Blocks start at even
-        // byte offsets: the copy is 2-byte aligned, and gfx950 runs global
-        // memory in unaligned-access mode, so it is still one dwordx3 load.
+        // One dword-aligned 12-byte load holding the lane's 8 bytes of qs: from
+        // byte 0 of the block (+ 8 h) for an even block, from 2 bytes before
+        // it for an odd one (rows start on dwords and hold whole pairs of
+        // blocks, so the load stays inside the row).  The lanes with h = 0
+        // get the block's scale with it.
         constexpr int kBlock = kType == kQ8_0 ? 34 : 18;
         const int h = kType == kQ8_0 ? g : (g & 1);  // which 8 bytes of qs
-        const unsigned char* p = wrow + static_cast<long long>(kBlock) * kb + (h ? 8 * h - 2 : 0);
-        __builtin_memcpy(w.u, p, 12);
+        const unsigned char* p = wrow + static_cast<long long>(kBlock) * kb + 8 * h - 2 * (kb & 1);
+        const unsigned* const q = reinterpret_cast<const unsigned*>(p);
+        w.u[0] = q[0];
+        w.u[1] = q[1];
+        w.u[2] = q[2];
     }
 }
 
@@ -192,9 +314,9 @@ __device__ __forceinline__ void load_w(WRaw<kType>& w, const unsigned char* wrow
 // by the block scale where there is one) and the block scale.
 template <int kType>
 __device__ __forceinline__ void decode_w(const WRaw<kType>& w, int kb, int g, bf16x8 (&b)[Fmt<kType>::kN],
-                                         float& d)
+                                         unsigned& d)
 {
-    d = 1.0f;
+    d = 0;
     if constexpr (kType == kF32) {
         const unsigned u[8] = {w.a.x, w.a.y, w.a.z, w.a.w, w.b.x, w.b.y, w.b.z, w.b.w};
 #pragma unroll
@@ -217,7 +339,7 @@ __device__ __forceinline__ void decode_w(const WRaw<kType>& w, int kb, int g, bf
     } else if constexpr (kType == kQ6_K) {
         const int k = kb & 3;
         const int sc = static_cast<signed char>(w.sd & 0xFFu);
-        d = half_to_float(w.sd >> 16);
+        d = w.sd >> 16;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const unsigned lo = (w.ql[e >> 2] >> (8 * (e & 3))) & 0xFFu;
@@ -229,11 +351,12 @@ __device__ __forceinline__ void decode_w(const WRaw<kType>& w, int kb, int g, bf
             b[1][e] = p1;
         }
     } else {
-        (void)kb;
-        const int h = kType == kQ8_0 ? g : (g & 1);
-        d = half_to_float(__shfl(w.u[0], threadIdx.x & 15) & 0xFFFFu);
-        const unsigned q[2] = {h ? w.u[1] : (w.u[0] >> 16) | (w.u[1] << 16),
-                               h ? w.u[2] : (w.u[1] >> 16) | (w.u[2] << 16)};
+        // the scale from the row's lane of g = 0; the 8 bytes at byte 2 of the
+        // load for an even block, at byte 4 for an odd one
+        const bool odd = kb & 1;
+        d = static_cast<unsigned>(__shfl(odd ? w.u[0] >> 16 : w.u[0], threadIdx.x & 15)) & 0xFFFFu;
+        const unsigned q[2] = {odd ? w.u[1] : (w.u[0] >> 16) | (w.u[1] << 16),
+                               odd ? w.u[2] : (w.u[1] >> 16) | (w.u[2] << 16)};
         // Each byte u (Q4_0: the nibble masked in place; Q8_0: the byte with
         // its sign bit flipped, q + 128) becomes the float 2^23 + u by one
         // byte permute into the mantissa of 2^23 (0x4B000000), and one
@@ -253,28 +376,52 @@ __device__ __forceinline__ void decode_w(const WRaw<kType>& w, int kb, int g, bf
     }
 }
 
-// One block's products for one (row subtile, token subtile) tile: acc (+)=
-// the products of pieces (b_i, x_p) with i + p <= 2, smallest terms first,
-// scaled by the block scale where there is one.
+// Weight c of a row, as the reference dequantises it.
 template <int kType>
-__device__ __forceinline__ void tile_products(const bf16x8 (&a)[3], const bf16x8 (&b)[Fmt<kType>::kN], float d,
-                                              floatx4& acc)
+__device__ __forceinline__ float weight_at(const unsigned char* wrow, int c)
 {
-    floatx4 t = Fmt<kType>::kScaled ? floatx4{0.f, 0.f, 0.f, 0.f} : acc;
-    if constexpr (Fmt<kType>::kN >= 3) t = mfma(a[0], b[2], t);
-    if constexpr (Fmt<kType>::kN >= 2) {
-        t = mfma(a[1], b[1], t);
-        t = mfma(a[0], b[1], t);
-    }
-    t = mfma(a[2], b[0], t);
-    t = mfma(a[1], b[0], t);
-    t = mfma(a[0], b[0], t);
-    if constexpr (Fmt<kType>::kScaled) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = fmaf(d, t[q], acc[q]);
+    const auto half_at = [](const unsigned char* p) { return half_to_float(p[0] | (p[1] << 8)); };
+    if constexpr (kType == kF32) {
+        return reinterpret_cast<const float*>(wrow)[c];
+    } else if constexpr (kType == kF16) {
+        return half_at(wrow + 2LL * c);
+    } else if constexpr (kType == kQ8_0) {
+        const unsigned char* const b = wrow + 34LL * (c >> 5);
+        return static_cast<float>(static_cast<signed char>(b[2 + (c & 31)])) * half_at(b);
+    } else if constexpr (kType == kQ4_0) {
+        const unsigned char* const b = wrow + 18LL * (c >> 5);
+        const int q = b[2 + (c & 15)] >> ((c & 16) ? 4 : 0) & 15;
+        return static_cast<float>(q - 8) * half_at(b);
     } else {
-        acc = t;
+        const unsigned char* const b = wrow + 210LL * (c >> 8);
+        const int h = c >> 7 & 1, k = c >> 5 & 3, l = c & 31;
+        const int lo = b[64 * h + 32 * (k & 1) + l] >> (k < 2 ? 0 : 4) & 15, hi = b[128 + 32 * h + l] >> (2 * k) & 3;
+        const float sc = static_cast<float>(static_cast<signed char>(b[192 + 8 * h + 2 * k + (l >> 4)]));
+        return half_at(b + 208) * sc * static_cast<float>((lo | hi << 4) - 32);
     }
+}
+
+// Pieces of an infinite operand can cancel to a NaN (inf - inf, 0 * inf), and a
+// block's unscaled sum can pass the largest float, where the products
+// themselves do neither: a sum that is not finite is taken again in plain
+// fp32 over columns [c0, c1), x from its row or from the planes.
+template <int kType, class X>
+__device__ __forceinline__ float plain_sum(const unsigned char* wrow, int c0, int c1, X&& x_at)
+{
+    float s = 0.f;
+#pragma unroll 1
+    for (int c = c0; c < c1; ++c) s += weight_at<kType>(wrow, c) * x_at(c);
+    return s;
+}
+
+__device__ __forceinline__ float plane_value(const unsigned char* xs, int t, int c, int n_blk)
+{
+    float v = 0.f;
+#pragma unroll
+    for (int pl = 2; pl >= 0; --pl)
+        v += static_cast<float>(*reinterpret_cast<const __bf16*>(
+            xs + plane_chunk(t >> 4, c >> 5, pl, n_blk) + 16 * (16 * (c >> 3 & 3) + (t & 15)) + 2 * (c & 7)));
+    return v;
 }
 
 // The segment holding a row: selected field by field (an index into the
@@ -285,7 +432,8 @@ struct RowSeg {
     long long stride;
     int row;  // within the segment
 };
-__device__ __forceinline__ RowSeg row_seg(const SplitParams& p, int row)
+template <class Params>
+__device__ __forceinline__ RowSeg row_seg(const Params& p, int row)
 {
     RowSeg r{p.seg[0].w, p.seg[0].out, p.seg[0].out_stride, row};
     int cur = 0;  // the segment r is in so far; only its successor can take the row
@@ -301,8 +449,446 @@ __device__ __forceinline__ RowSeg row_seg(const SplitParams& p, int row)
     return r;
 }
 
+// The lane's 8 weights of an F32 block.
+template <int kType>
+__device__ __forceinline__ split_f32x8 float_w(const WRaw<kType>& w)
+{
+    split_f32x8 v{};
+    if constexpr (kType == kF32) {
+        const unsigned u[8] = {w.a.x, w.a.y, w.a.z, w.a.w, w.b.x, w.b.y, w.b.z, w.b.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = __builtin_bit_cast(float, u[e]);
+    }
+    return v;
+}
+
+// One block's products for kR row subtiles: acc (+)= the products of pieces
+// (x_p, b_i) with i + p <= 2, smallest terms first, scaled by the block scale
+// (the bits of a half) where there is one.  Each block is summed from zero:
+// carried through the matrix cores from block to block, F16 sums were 2.2e-7
+// off fp64 at 2048 columns against 1e-7.
+template <int kType, int kR>
+__device__ __forceinline__ void block_products(const bf16x8 (&x)[3], const bf16x8 (&b)[kR][Fmt<kType>::kN],
+                                               const unsigned (&d)[kR], floatx4 (&acc)[kR])
+{
+    constexpr int kN = Fmt<kType>::kN;
+    floatx4 t[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) t[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (kN >= 3) {
+#pragma unroll
+        for (int r = 0; r < kR; ++r) t[r] = mfma(x[0], b[r][kN - 1], t[r]);
+    }
+    if constexpr (kN >= 2) {
+#pragma unroll
+        for (int r = 0; r < kR; ++r) t[r] = mfma(x[1], b[r][1], t[r]);
+#pragma unroll
+        for (int r = 0; r < kR; ++r) t[r] = mfma(x[0], b[r][1], t[r]);
+    }
+#pragma unroll
+    for (int pl = 2; pl >= 0; --pl)
+#pragma unroll
+        for (int r = 0; r < kR; ++r) t[r] = mfma(x[pl], b[r][0], t[r]);
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+        if constexpr (Fmt<kType>::kScaled) {
+            const float s = half_to_float(d[r]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) acc[r][q] = fmaf(s, t[r][q], acc[r][q]);
+        } else {
+            acc[r] += t[r];
+        }
+    }
+}
+
+// Row j of row subtile `sub`: row 16 sub + j of the segments laid end to end,
+// or, paired, gate row 8 sub + j (j < 8) and up row 8 sub + j - 8.  Past the
+// end: the last row, not ok.
+struct TileRow : RowSeg {
+    bool ok;
+};
+__device__ __forceinline__ TileRow tile_row(const ProductParams& p, int sub, int j)
+{
+    TileRow r;
+    if (p.pair) {
+        const int row = 8 * sub + (j & 7), last = p.seg[0].rows - 1;
+        const bool up = j >= 8;
+        r.w = up ? p.seg[1].w : p.seg[0].w;
+        r.out = up ? p.seg[1].out : p.seg[0].out;
+        r.stride = up ? p.seg[1].out_stride : p.seg[0].out_stride;
+        r.row = min(row, last);
+        r.ok = row <= last;
+    } else {
+        const int row = 16 * sub + j;
+        static_cast<RowSeg&>(r) = row_seg(p, min(row, p.total_rows - 1));
+        r.ok = row < p.total_rows;
+    }
+    return r;
+}
+
+// Paired, after the raw products: lanes j < 8 hold token t's gate sums of the
+// eight rows 8 sub .. + 7, lanes j + 8 their up sums: silu(gate) * up into the
+// planes of the down projection's input, where those eight columns of the
+// token are one 16-byte piece.  All lanes call it.
+__device__ __forceinline__ void store_gated(const ProductParams& p, float sum, int t, int row, bool ok, int j)
+{
+    const float up = __shfl(sum, (threadIdx.x & 63) ^ 8);
+    if (j >= 8 || !ok) return;
+    float v[8] = {gated(sum, up), 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    bf16x8 x[3];
+    split_any(v, x);
+    const int slot = 16 * (row >> 3 & 3) + (t & 15), n_blk = p.seg[0].rows >> 5;
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl)
+        *reinterpret_cast<__bf16*>(p.hs + plane_chunk(t >> 4, row >> 5, pl, n_blk) + 16 * slot + 2 * (row & 7)) =
+            x[pl][0];
+}
+
+// ---- direct --------------------------------------------------------------------
+// kR row subtiles x one token tile per workgroup, K over its 8 waves (wave w
+// blocks w, w + 8, ...; the waves' sums meet in LDS in wave order).  Every
+// load a wave makes for 2048 columns is in flight at once: the launch is one
+// memory round trip, then vector work (splitting x, about 44 operations a
+// block, and dequantising, about 30 a subtile) that bounds it.  With kXNormRows x is
+// multiplied by the norm's weights before it is split and the sums by the
+// row's 1 / rms at the end, so that no launch goes before it.  Q8_0, 12
+// tokens, TinyLlama's layer (kernel trace): rmsnorm + Q/K/V 11.4 us, W_o 8.8,
+// rmsnorm + gate | up + SwiGLU 15.0, W_down 12.3, where matrix-vector launches
+// (weights read once per 2 to 6 vectors) took 56, 39, 78 and 142 us.  16 waves of
+// 128 registers spilled; two row subtiles where one round of workgroups takes
+// one cost 2-3 us more; loads behind branches made every block wait for all of
+// them (2560 x 2048, Q8_0, 3 tokens, 6.9 against 6.4 us).  F32 weights from fp32 rows take the fp32 matrix cores
+// instead (kFp32: lane group g the columns 8 g + e of step e, each block summed
+// from zero): one token tile does not repay splitting both operands (2560 x
+// 2048, 3 tokens, 9.2 us split, 8.4 so; F16 with three row subtiles 12.9
+// split, 15.1 so).
+enum XSource { kXRows, kXNormRows, kXPlanes };
+
+template <int kType, int kR, int kSrc, int kDepth>
+__global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const ProductParams p)
+{
+    constexpr int kN = Fmt<kType>::kN;
+    constexpr bool kNorm = kSrc == kXNormRows;
+    constexpr bool kFp32 = kSrc != kXPlanes && kType == kF32;
+    constexpr int kCombos = 4 * kR;
+    __shared__ float s_red[kWaves][kCombos][64];
+    __shared__ float s_ss[kWaves][16];
+    __shared__ __align__(16) float s_norm[kNorm ? kProductMaxNorm : 4];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int j = lane & 15, g = lane >> 4;
+    const int n_blk = p.cols >> 5, tile = blockIdx.y;
+    const int sub0 = blockIdx.x * kR;
+    // blocks wave + kWaves i, i < nb
+    const int nb = wave < n_blk ? (n_blk - wave + kWaves - 1) / kWaves : 0;
+    const unsigned char* wrow[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+        const TileRow rs = tile_row(p, sub0 + r, j);
+        wrow[r] = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
+    }
+    const float* const xrow = p.x + static_cast<long long>(min(16 * tile + j, p.n - 1)) * p.x_stride + 8 * g;
+
+    struct Stage {
+        WRaw<kType> w[kR];
+        u32x4 x[kSrc == kXPlanes ? 3 : 2];  // eight floats, or their planes
+    } st[kDepth];
+    // (past the wave's last block that one again, never used: no load sits
+    // behind a branch, where the compiler would wait for all in flight)
+    const auto load = [&](Stage& t, int i) __attribute__((always_inline)) {
+        const int kb = min(wave + kWaves * min(i, max(nb - 1, 0)), n_blk - 1);
+        const unsigned char* const src =
+            kSrc == kXPlanes ? p.xs + plane_chunk(tile, kb, 0, n_blk) + 16 * lane
+                             : reinterpret_cast<const unsigned char*>(xrow + 32 * kb);
+#pragma unroll
+        for (int i2 = 0; i2 < (kSrc == kXPlanes ? 3 : 2); ++i2)
+            t.x[i2] = *reinterpret_cast<const u32x4*>(src + (kSrc == kXPlanes ? 1024 : 16) * i2);
+#pragma unroll
+        for (int r = 0; r < kR; ++r) load_w<kType>(t.w[r], wrow[r], kb, g);
+    };
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+        load(st[d], d);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kNorm) {
+        for (int c = 4 * threadIdx.x; c < p.cols; c += 4 * kWaves * 64)
+            *reinterpret_cast<float4*>(s_norm + c) = *reinterpret_cast<const float4*>(p.norm_w + c);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the loads above stay in flight
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
+    floatx4 acc[kR];
+#pragma unroll
+    for (int r = 0; r < kR; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float ss = 0.f;
+    const auto block = [&](const Stage& t, int i) __attribute__((always_inline)) {
+        const int kb = wave + kWaves * i;
+        split_f32x8 v;
+        if constexpr (kSrc != kXPlanes) {
+            const float4 xa = __builtin_bit_cast(float4, t.x[0]), xb = __builtin_bit_cast(float4, t.x[1]);
+            v = split_f32x8{xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+            if constexpr (kNorm) {
+                const float4* const nw = reinterpret_cast<const float4*>(s_norm + 32 * kb + 8 * g);
+                const float4 na = nw[0], nb4 = nw[1];
+                ss += sum_sq4(xa) + sum_sq4(xb);
+                v *= split_f32x8{na.x, na.y, na.z, na.w, nb4.x, nb4.y, nb4.z, nb4.w};
+            }
+        }
+        if constexpr (kFp32) {
+            floatx4 sum[kR];
+            split_f32x8 w[kR];
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                sum[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+                w[r] = float_w<kType>(t.w[r]);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+#pragma unroll
+                for (int r = 0; r < kR; ++r)
+                    sum[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], w[r][e], sum[r], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < kR; ++r) acc[r] += sum[r];
+        } else {
+            bf16x8 x[3];
+            if constexpr (kSrc == kXPlanes) {
+#pragma unroll
+                for (int pl = 0; pl < 3; ++pl) x[pl] = __builtin_bit_cast(bf16x8, t.x[pl]);
+            } else {
+                split3x8(v, x[0], x[1], x[2]);
+            }
+            bf16x8 b[kR][kN];
+            unsigned d[kR];
+#pragma unroll
+            for (int r = 0; r < kR; ++r) decode_w<kType>(t.w[r], kb, g, b[r], d[r]);
+            block_products<kType, kR>(x, b, d, acc);
+        }
+    };
+    int i0 = 0;
+    for (; i0 + kDepth < nb; i0 += kDepth) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            block(st[d], i0 + d);
+            __builtin_amdgcn_sched_barrier(0);
+            load(st[d], i0 + d + kDepth);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d)
+        if (i0 + d < nb) block(st[d], i0 + d);  // uniform
+#pragma unroll
+    for (int r = 0; r < kR; ++r)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s_red[wave][4 * r + q][lane] = acc[r][q];
+    if constexpr (kNorm) {
+        ss += __shfl_xor(ss, 16);
+        ss += __shfl_xor(ss, 32);
+        if (g == 0) s_ss[wave][j] = ss;
+    }
+    __syncthreads();
+    // combination c: token 4 g + c % 4 of row subtile c / 4
+#pragma unroll
+    for (int c0 = 0; c0 < kCombos; c0 += kWaves) {
+        const int c = c0 + wave, t = 16 * tile + 4 * g + (c & 3);
+        if (c >= kCombos) return;
+        float sum = s_red[0][c][lane];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) sum += s_red[w][c][lane];
+        const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
+        const bool ok = rs.ok && t < p.n;
+        if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
+            const unsigned char* const wr = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
+            const float* const xr = p.x + t * p.x_stride;
+            sum = plain_sum<kType>(wr, 0, p.cols, [&](int col) {
+                return kSrc == kXPlanes ? plane_value(p.xs, t, col, n_blk) : kNorm ? xr[col] * s_norm[col] : xr[col];
+            });
+        }
+        if constexpr (kNorm) {
+            float s2 = s_ss[0][4 * g + (c & 3)];
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) s2 += s_ss[w][4 * g + (c & 3)];
+            sum *= 1.0f / sqrtf(s2 / static_cast<float>(p.cols) + p.eps);
+        }
+        if (ok && rs.out) {
+            float* const o = rs.out + rs.row + t * rs.stride;
+            *o = p.add ? *o + sum : sum;
+        }
+        if (p.pair) store_gated(p, sum, t, rs.row, ok, j);
+    }
+}
+
+// ---- resident ------------------------------------------------------------------
+// A workgroup of 8 waves holds the decoded weights of kR row subtiles x one K
+// range (up to 2048 columns, one slice of kSlice blocks per wave) in registers
+// and streams the x planes of its share of the token tiles past them: the
+// weights are read and dequantised once per share, and nothing but the planes
+// moves per tile.  Each wave keeps kRing blocks of x ahead in registers; the
+// waves' sums meet in LDS.  Bound by the planes' way into the CU: a tile is 196 KB per
+// workgroup, 1.6 us at the ~50 B a clock a CU takes from L2, against 0.96 us of
+// matrix work with three subtiles (measured per tile: 1.77 / 1.94 / 2.1 us with 1 / 2
+// / 3 subtiles).  All workgroups walk their tiles in the same order, so an
+// XCD's share of them meets in its L2; a flat split of (group, tile) units over
+// the CUs did not (4 us a tile).  An LDS ring filled by direct loads was slower
+// (1.5 us + 0.31 a subtile: written and read, x passes the LDS port twice), and
+// so were loads of the weights' 8 bytes at their own 2-byte alignment (gate |
+// up, 64 tokens, 49 against 22 us).  Q4_0, 11264 x 2048 with the planes'
+// launch, tiled / resident: 65 tokens 37 / 22 us, 160 55 / 34, 512 94 / 80.
+template <int kType, int kR, int kSlice>
+__global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const ProductParams p)
+{
+    constexpr int kN = Fmt<kType>::kN;
+    constexpr int kCombos = 4 * kR;                         // (row subtile, token of four) sums per lane
+    constexpr int kOuts = (kCombos + kWaves - 1) / kWaves;  // of which each wave finishes
+    __shared__ float s_red[2][kWaves][kCombos][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int j = lane & 15, g = lane >> 4;
+    const int n_blk = p.cols >> 5;
+    const int tiles = p.n_tiles;
+    int buf = 0;
+    {
+        const int share = blockIdx.x % p.shares, group = blockIdx.x / p.shares;
+        const int tile0 = static_cast<int>(static_cast<long long>(tiles) * share / p.shares);
+        const int here = static_cast<int>(static_cast<long long>(tiles) * (share + 1) / p.shares) - tile0;
+        const int z = group / p.row_groups, sub0 = (group % p.row_groups) * kR;
+        // this wave's blocks [kb0, kb0 + nb) of K range z
+        const int kb_lo = z * p.blk_per_split, kb_hi = min(kb_lo + p.blk_per_split, n_blk);
+        const int per_wave = (kb_hi - kb_lo + 2 * kWaves - 1) / (2 * kWaves) * 2;
+        const int kb0 = kb_lo + wave * per_wave;
+        const int nb = max(0, min(per_wave, kb_hi - kb0));
+        // past the slice: a block of the same parity, loaded but not used
+        const auto block_of = [&](int b) { return min(kb0 + b, kb_hi - 2 + (b & 1)); };
+        bf16x8 ring[kRing][3];
+        const auto load_x = [&](int b, int tile) __attribute__((always_inline)) {
+            const unsigned char* const src = p.xs + plane_chunk(tile, block_of(b), 0, n_blk) + 16 * lane;
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) ring[b % kRing][pl] = *reinterpret_cast<const bf16x8*>(src + 1024 * pl);
+        };
+
+        // the row group's weights, all requested at once, then the first
+        // tile's x; decoded into registers for every tile of the group
+        bf16x8 held[kR][kSlice][kN];
+        unsigned scale[kR][kSlice / 2];  // two block scales a word, as halves
+        {
+            WRaw<kType> raw[kR][kSlice];
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                const TileRow rs = tile_row(p, sub0 + r, j);
+                const unsigned char* const wrow = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
+#pragma unroll
+                for (int b = 0; b < kSlice; ++b) load_w<kType>(raw[r][b], wrow, block_of(b), g);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int b = 0; b < kRing; ++b) load_x(b, tile0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < kR; ++r)
+#pragma unroll
+                for (int b = 0; b < kSlice; ++b) {
+                    unsigned d;
+                    decode_w<kType>(raw[r][b], block_of(b), g, held[r][b], d);
+                    scale[r][b / 2] = b % 2 ? scale[r][b / 2] | (d << 16) : d;
+                }
+        }
+
+        // where this wave's finished sums go: tokens 4 g + c % 4 of row j of
+        // subtile c / 4 for its combinations c
+        float* out[kOuts];
+        long long stride[kOuts];
+        bool row_ok[kOuts];
+#pragma unroll
+        for (int i = 0; i < kOuts; ++i) {
+            const int c = wave + kWaves * i;
+            const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
+            row_ok[i] = c < kCombos && rs.ok;
+            if (p.part) {
+                out[i] = p.part + static_cast<long long>(z) * p.n * p.total_rows + 16 * (sub0 + (c >> 2)) + j;
+                stride[i] = p.total_rows;
+            } else {
+                out[i] = rs.out ? rs.out + rs.row : nullptr;
+                stride[i] = rs.stride;
+            }
+        }
+
+        const auto tile_step = [&](int tile, auto next) __attribute__((always_inline)) {
+            constexpr bool kNext = decltype(next)::value;
+            floatx4 acc[kR];
+#pragma unroll
+            for (int r = 0; r < kR; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+            const auto block_step = [&](int b) __attribute__((always_inline)) {
+                if (b >= nb) return;  // uniform
+                const bf16x8(&x)[3] = ring[b % kRing];
+                bf16x8 w[kR][kN];
+                unsigned d[kR];
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    d[r] = b % 2 ? scale[r][b / 2] >> 16 : scale[r][b / 2] & 0xFFFFu;
+#pragma unroll
+                    for (int i = 0; i < kN; ++i) w[r][i] = held[r][b][i];
+                }
+                block_products<kType, kR>(x, w, d, acc);
+            };
+#pragma unroll
+            for (int b = 0; b < kSlice; ++b) {
+                block_step(b);
+                __builtin_amdgcn_sched_barrier(0);
+                if (b + kRing < kSlice)
+                    load_x(b + kRing, tile);
+                else if constexpr (kNext)
+                    load_x(b + kRing - kSlice, tile + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the waves' sums in wave order; two buffers, so one barrier a tile
+#pragma unroll
+            for (int r = 0; r < kR; ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s_red[buf][wave][4 * r + q][lane] = acc[r][q];
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the copies ahead stay in flight
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < kOuts; ++i) {
+                const int c = min(wave + kWaves * i, kCombos - 1);
+                float sum = s_red[buf][0][c][lane];
+#pragma unroll
+                for (int w = 1; w < kWaves; ++w) sum += s_red[buf][w][c][lane];
+                const int t = 16 * tile + 4 * g + (c & 3);
+                const bool ok = row_ok[i] && t < p.n;
+                if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
+                    const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
+                    sum = plain_sum<kType>(rs.w + static_cast<long long>(rs.row) * p.row_bytes, 32 * kb_lo, 32 * kb_hi,
+                                           [&](int col) { return plane_value(p.xs, t, col, n_blk); });
+                }
+                if (ok && out[i]) {
+                    float* const o = out[i] + t * stride[i];
+                    *o = p.add && !p.part ? *o + sum : sum;
+                }
+                if (p.pair && wave + kWaves * i < kCombos)
+                    store_gated(p, sum, t, 8 * (sub0 + (c >> 2)) + (j & 7), ok, j);
+            }
+            asm volatile("" ::: "memory");
+            buf ^= 1;
+        };
+#pragma unroll 1
+        for (int i = 0; i + 1 < here; ++i) tile_step(tile0 + i, std::true_type{});
+        tile_step(tile0 + here - 1, std::false_type{});
+    }
+}
+
+// ---- tiled ---------------------------------------------------------------------
+// A workgroup of 4 waves owns 64 kRW weight rows x 64 tokens (4 token tiles);
+// wave w owns rows 16 kRW w .. + 16 kRW - 1 for all 64 tokens.  The x blocks
+// pass through a ring of three LDS stages (12 KiB each) filled by direct
+// loads two blocks ahead; each wave loads its rows' weights three blocks
+// ahead.  Bound by its barrier per block and LDS reads; kept where the
+// resident product holds too few rows or needs several K ranges (512 tokens,
+// us, tiled / resident: F16 11264 x 2048 105 / 123, F32 155 / 191, Q8_0
+// 2048 x 5632 61 / 69; at 160 tokens 57 / 55, 82 / 76, 35 / 33).
 template <int kType, int kRW>
-__global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitParams p)
+__global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const ProductParams p)
 {
     // The ring's stages as separate arrays, so that the compiler sees that a
     // stage being read is not the one a copy in flight writes.
@@ -317,11 +903,12 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
     const unsigned L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     const unsigned ty = L % gridDim.y, rest = L / gridDim.y;
     const unsigned tx = rest % gridDim.x, tz = rest / gridDim.x;
-    const int row0 = (tx * kWaves + wave) * 16 * kRW;
+    const int n_blk = p.cols >> 5;
+    const int row0 = (tx * kTileWaves + wave) * 16 * kRW;
     const int s0 = ty * kTW;  // first token subtile
     // K range of this workgroup: blocks [kb_lo, kb_hi) (grid z splits K)
     const int kb_lo = tz * p.blk_per_split;
-    const int kb_hi = min(kb_lo + p.blk_per_split, p.cols >> 5);
+    const int kb_hi = min(kb_lo + p.blk_per_split, n_blk);
 
     // this lane's weight row in each row subtile (the last row for rows past
     // the end: loaded, never stored)
@@ -343,12 +930,12 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
         for (int i = 0; i < kChunksPerWave; ++i) {
             const int c = kChunksPerWave * wave + i;
             __builtin_amdgcn_global_load_lds(
-                (global_ptr)(p.xs + plane_chunk(kb, c / kTW, s0, p.n_sub) + 1024 * (c % kTW) + 16 * lane),
+                (global_ptr)(p.xs + plane_chunk(s0 + c % kTW, kb, c / kTW, n_blk) + 16 * lane),
                 (lds_ptr)(stage_base(stage) + 1024 * c), 16, 0, 0);
         }
     };
     auto load_ws = [&](WRaw<kType> (&wr)[kRW], int kb) __attribute__((always_inline)) {
-        kb = min(kb, kb_hi - 1);
+        kb = kb < kb_hi ? kb : kb_hi - 2 + (kb & 1);
 #pragma unroll
         for (int r = 0; r < kRW; ++r) load_w<kType>(wr[r], wrow[r], kb, g);
     };
@@ -404,7 +991,7 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
             // the row subtiles' weights first, then the token subtiles one
             // at a time (their x pieces read from LDS just before use)
             bf16x8 b[kRW][Fmt<kType>::kN];
-            float d[kRW];
+            unsigned d[kRW];
 #pragma unroll
             for (int r = 0; r < kRW; ++r) decode_w<kType>(wr_this[r], kb, g, b[r], d[r]);
 #pragma unroll
@@ -414,7 +1001,12 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
                 for (int pl = 0; pl < 3; ++pl)
                     a[pl] = *reinterpret_cast<const bf16x8*>(stage_base(u) + (pl * kTW + s) * 1024 + 16 * lane);
 #pragma unroll
-                for (int r = 0; r < kRW; ++r) tile_products<kType>(a, b[r], d[r], acc[r][s]);
+                for (int r = 0; r < kRW; ++r) {
+                    floatx4 one[1] = {acc[r][s]};
+                    block_products<kType, 1>(a, reinterpret_cast<const bf16x8(&)[1][Fmt<kType>::kN]>(b[r]),
+                                             reinterpret_cast<const unsigned(&)[1]>(d[r]), one);
+                    acc[r][s] = one[0];
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -422,7 +1014,7 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
         __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll 1
-    for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += kRing) {
+    for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += kStages) {
         iteration(kb0, wr0, 0, 2);
         iteration(kb0 + 1, wr1, 1, 0);
         iteration(kb0 + 2, wr2, 2, 1);
@@ -431,7 +1023,7 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
     __builtin_amdgcn_s_waitcnt(0);
 
     // lane (g, j) holds tokens 16 (s0 + s) + 4 g + q of row row0 + 16 r + j;
-    // with K split, the sums go to part[z][t][row] for split_reduce_kernel
+    // with K split, the sums go to part[z][t][row] for range_sum_kernel
 #pragma unroll
     for (int r = 0; r < kRW; ++r) {
         const int row = row0 + 16 * r + j;
@@ -464,7 +1056,7 @@ __global__ __launch_bounds__(kThreads) void split_product_kernel(const SplitPara
 
 // out[t][row] (+)= sum over the K splits z, in order, of part[z][t][row]:
 // one thread per (t, row).
-__global__ __launch_bounds__(kThreads) void split_reduce_kernel(const SplitParams p)
+__global__ __launch_bounds__(kThreads) void range_sum_kernel(const ProductParams p)
 {
     const long long id = static_cast<long long>(blockIdx.x) * kThreads + threadIdx.x;
     if (id >= static_cast<long long>(p.n) * p.total_rows) return;
@@ -477,72 +1069,239 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const SplitParam
     *o = p.add ? *o + sum : sum;
 }
 
-template <int kType, int kRW>
-hipError_t launch_product(const SplitParams& p, hipStream_t s)
+// Row subtiles per workgroup that the registers hold: a direct workgroup's raw
+// weights, a resident one's decoded weights (4 registers per block, piece and
+// subtile).
+constexpr int direct_rows(int type) { return type == kQ6_K ? 2 : kMaxRows; }
+constexpr int resident_rows(int type) { return type == kF32 ? 1 : type == kF16 || type == kQ6_K ? 2 : kMaxRows; }
+
+template <int kType, int kR, int kDepth>
+hipError_t launch_direct_depth(const ProductParams& p, hipStream_t s)
 {
-    const dim3 grid(static_cast<unsigned>((p.total_rows + 64 * kRW - 1) / (64 * kRW)),
-                    static_cast<unsigned>(p.n_sub / kTW), static_cast<unsigned>(p.k_splits));
-    hipLaunchKernelGGL((split_product_kernel<kType, kRW>), grid, dim3(kThreads), 0, s, p);
+    const dim3 grid(static_cast<unsigned>(p.row_groups), static_cast<unsigned>(p.n_tiles)), block(kWaves * 64);
+    if (p.planes)
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXPlanes, kDepth>), grid, block, 0, s, p);
+    else if (p.norm_w)
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXNormRows, kDepth>), grid, block, 0, s, p);
+    else
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXRows, kDepth>), grid, block, 0, s, p);
+    return hipGetLastError();
+}
+
+// Blocks in flight per wave: all of 2048 columns with one row subtile (fewer
+// where the row has fewer: a load past the end is made, not used), else four,
+// which is what the registers hold beside three subtiles.
+template <int kType, int kR>
+hipError_t launch_direct(const ProductParams& p, hipStream_t s)
+{
+    if constexpr (kR == 1) {
+        const int blocks = (p.cols / 32 + kWaves - 1) / kWaves;
+        return blocks <= 2   ? launch_direct_depth<kType, 1, 2>(p, s)
+               : blocks <= 4 ? launch_direct_depth<kType, 1, 4>(p, s)
+                             : launch_direct_depth<kType, 1, 8>(p, s);
+    } else if constexpr (kR <= direct_rows(kType)) {
+        return launch_direct_depth<kType, kR, 4>(p, s);
+    } else {
+        return hipErrorInvalidValue;
+    }
+}
+
+template <int kType, int kR>
+hipError_t launch_resident(const ProductParams& p, hipStream_t s)
+{
+    if constexpr (kR <= resident_rows(kType)) {
+        const dim3 grid(static_cast<unsigned>(p.row_groups * p.k_splits * p.shares)), block(kWaves * 64);
+        if (p.blk_per_split <= 4 * kWaves)
+            hipLaunchKernelGGL((resident_product_kernel<kType, kR, 4>), grid, block, 0, s, p);
+        else
+            hipLaunchKernelGGL((resident_product_kernel<kType, kR, kMaxSlice>), grid, block, 0, s, p);
+        return hipGetLastError();
+    } else {
+        return hipErrorInvalidValue;
+    }
+}
+
+template <int kType, int kR>
+hipError_t launch_tiled(const ProductParams& p, hipStream_t s)
+{
+    const dim3 grid(static_cast<unsigned>(p.row_groups), static_cast<unsigned>(p.n_tiles / kTW),
+                    static_cast<unsigned>(p.k_splits));
+    hipLaunchKernelGGL((tiled_product_kernel<kType, kR>), grid, dim3(kTileThreads), 0, s, p);
     return hipGetLastError();
 }
 
 template <int kType>
-hipError_t launch_typed(const SplitParams& p, hipStream_t s)
+hipError_t launch_typed(const ProductParams& p, hipStream_t s)
 {
-    hipError_t err;
-    switch (p.rows_per_wave) {
-    case 1: err = launch_product<kType, 1>(p, s); break;
-    case 2: err = launch_product<kType, 2>(p, s); break;
-    default: err = launch_product<kType, 4>(p, s); break;
-    }
+    const int r = p.rows_per_group;
+    if (p.kind == kProductDirect)
+        return r == 1   ? launch_direct<kType, 1>(p, s)
+               : r == 2 ? launch_direct<kType, 2>(p, s)
+                        : launch_direct<kType, 3>(p, s);
+    const hipError_t err = p.kind == kProductTiled ? (r == 1 ? launch_tiled<kType, 1>(p, s) : launch_tiled<kType, 2>(p, s))
+                           : r == 1                ? launch_resident<kType, 1>(p, s)
+                           : r == 2                ? launch_resident<kType, 2>(p, s)
+                                                   : launch_resident<kType, 3>(p, s);
     if (err != hipSuccess || !p.part || p.defer_reduce) return err;
     const long long n = static_cast<long long>(p.n) * p.total_rows;
-    hipLaunchKernelGGL(split_reduce_kernel, dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, s, p);
+    hipLaunchKernelGGL(range_sum_kernel, dim3(static_cast<unsigned>((n + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                       s, p);
     return hipGetLastError();
 }
 
 }  // namespace
 
-size_t split_x_bytes(int n, int cols)
+void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p)
 {
-    return static_cast<size_t>(split_tokens(n)) * static_cast<size_t>(cols) * 6;
+    const int n_blk = p->cols / 32, sub = (p->total_rows + 15) / 16, tiles = (p->n + 15) / 16;
+    p->n_tiles = tiles;
+    p->k_splits = 1;
+    p->blk_per_split = n_blk;
+    p->shares = 1;
+    // Up to 16 tokens, or where the row subtiles and token tiles fit the CUs
+    // in one round: no launch for the planes.  As many rows per workgroup as
+    // bring the grid into one round (11264 x 2048, 3 tokens, 1 / 2 / 3
+    // subtiles: Q4_0 17.9 / 17.6 / 12.2 us); past that two, whose registers let
+    // a CU hold two workgroups (32000 rows 28.2 / 23.2 / 29.5).
+    if (tiles == 1 || static_cast<long long>(sub) * tiles <= n_cu) {
+        p->kind = kProductDirect;
+        int r = 1;
+        while (r < direct_rows(type) && static_cast<long long>((sub + r - 1) / r) * tiles > n_cu) ++r;
+        if (static_cast<long long>((sub + r - 1) / r) * tiles > n_cu) r = 2;
+        if (opt_rows > 0) r = std::min(opt_rows, direct_rows(type));
+        p->rows_per_group = r;
+        p->row_groups = (sub + r - 1) / r;
+        return;
+    }
+    const int ranges = (n_blk + kRangeBlocks - 1) / kRangeBlocks;
+    const bool tiled = p->n > 192 && type != kQ6_K && !p->pair &&
+                       (ranges > 1 || (type == kF16 && p->total_rows > 4096) || (type == kF32 && p->total_rows > 2048));
+    int splits = std::max(ranges, std::min(opt_k, n_blk / 2));
+    if (tiled) {
+        p->kind = kProductTiled;
+        p->n_tiles = (p->n + 16 * kTW - 1) / (16 * kTW) * kTW;
+        // Two row subtiles per wave where that gives half the CUs a
+        // workgroup; K cut until the grid holds about 2.5 workgroups per CU,
+        // ranges of at least 8 blocks.
+        const auto groups = [&](int r) { return (p->total_rows + 64LL * r - 1) / (64LL * r) * (p->n_tiles / kTW); };
+        int r = 2 * groups(2) >= n_cu ? 2 : 1;
+        if (opt_rows > 0) r = std::min(opt_rows, 2);
+        p->rows_per_group = r;
+        p->row_groups = (p->total_rows + 64 * r - 1) / (64 * r);
+        const long long target = 5LL * n_cu / 2;
+        splits = static_cast<int>(std::min<long long>((target + groups(r) - 1) / groups(r), n_blk / 8));
+        if (opt_k > 0) splits = std::min(opt_k, n_blk / 2);
+        splits = std::max(1, splits);
+    } else {
+        p->kind = kProductResident;
+        // The rows per workgroup and the shares of the token tiles with the
+        // least estimated time, in microseconds: per round of workgroups, the
+        // weights (3 + 1.5 per row subtile) and each token tile (1.6 to load
+        // its planes, 0.17 per row subtile not hidden behind that).
+        double best = 0;
+        const int most = resident_rows(type);
+        for (int r = 1; r <= most; ++r) {
+            if (opt_rows > 0 && r != std::min(opt_rows, most)) continue;
+            const long long groups = static_cast<long long>((sub + r - 1) / r) * splits;
+            for (int shares = 1; shares <= std::min(tiles, 8); ++shares) {
+                const int each = (tiles + shares - 1) / shares;
+                if (opt_tiles > 0 && shares < std::min(tiles, 8) && each > opt_tiles) continue;
+                const double rounds = static_cast<double>((groups * shares + n_cu - 1) / n_cu);
+                const double cost = rounds * (3.0 + 1.5 * r + each * (1.6 + 0.17 * r));
+                if (best == 0 || cost < best) {
+                    best = cost;
+                    p->rows_per_group = r;
+                    p->row_groups = (sub + r - 1) / r;
+                    p->shares = shares;
+                }
+            }
+        }
+    }
+    p->blk_per_split = (n_blk / 2 + splits - 1) / splits * 2;
+    p->k_splits = (n_blk + p->blk_per_split - 1) / p->blk_per_split;
 }
 
-size_t split_part_bytes(int n, int total_rows, int k_splits)
+size_t product_planes_bytes(int n, int cols)
+{
+    return static_cast<size_t>((n + 16 * kTW - 1) / (16 * kTW) * (16 * kTW)) * static_cast<size_t>(cols) * 6;
+}
+
+size_t product_part_bytes(int n, int total_rows, int k_splits)
 {
     return static_cast<size_t>(n) * static_cast<size_t>(total_rows) * static_cast<size_t>(k_splits) * sizeof(float);
 }
 
-int split_tokens(int n)
+namespace {
+bool a16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+}  // namespace
+
+hipError_t load_product_code()
 {
-    return (n + 16 * kTW - 1) / (16 * kTW) * (16 * kTW);
+    hipFuncAttributes a;
+    return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&norm_split_rows_kernel));
 }
 
-hipError_t launch_split_rows(const float* x, long long x_stride, int n, int cols, unsigned char* xs, hipStream_t s)
+hipError_t launch_split_rows(const float* x, long long x_stride, int n, int cols, bool gated, unsigned char* xs,
+                             hipStream_t s)
 {
-    if (n < 1 || cols < 32 || cols % 32 != 0 || x_stride % 4 != 0 || reinterpret_cast<uintptr_t>(x) % 16 != 0)
-        return hipErrorInvalidValue;
-    const int n_sub = split_tokens(n) / 16, n_blk = cols / 32;
-    const long long threads = static_cast<long long>(n_blk) * n_sub * 64;
-    hipLaunchKernelGGL(split_rows_kernel, dim3(static_cast<unsigned>((threads + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, s, x, x_stride, n, n_sub, n_blk, xs);
+    if (n < 1 || cols < 32 || cols % 32 != 0 || x_stride % 4 != 0 || !a16(x) || !a16(xs)) return hipErrorInvalidValue;
+    const int n_tiles = (n + 15) / 16, n_blk = cols / 32;
+    const long long threads = static_cast<long long>(n_blk) * n_tiles * 64;
+    const dim3 grid(static_cast<unsigned>((threads + kThreads - 1) / kThreads));
+    if (gated)
+        hipLaunchKernelGGL((split_rows_kernel<true>), grid, dim3(kThreads), 0, s, x, x_stride, n, n_tiles, n_blk, xs);
+    else
+        hipLaunchKernelGGL((split_rows_kernel<false>), grid, dim3(kThreads), 0, s, x, x_stride, n, n_tiles, n_blk, xs);
     return hipGetLastError();
 }
 
-hipError_t launch_split_product(int type, const SplitParams& p, hipStream_t s)
+hipError_t launch_norm_split_rows(float* x, const float* part, int k_splits, int n, int cols, const float* w, float eps,
+                                  unsigned char* xs, hipStream_t s)
 {
-    if (p.n < 1 || p.total_rows < 1 || p.cols < 32 || p.cols % 32 != 0 || (type == kQ6_K && p.cols % 256 != 0) ||
-        p.n_sub != split_tokens(p.n) / 16 || p.n_seg < 1 || p.n_seg > kGemvMaxSeg ||
-        p.row_bytes != static_cast<long long>(weight_row_bytes(type, p.cols)) ||
-        (p.rows_per_wave != 1 && p.rows_per_wave != 2 && p.rows_per_wave != 4) || p.k_splits < 1 ||
-        p.blk_per_split < 1 || static_cast<long long>(p.k_splits - 1) * p.blk_per_split >= p.cols / 32 ||
-        static_cast<long long>(p.k_splits) * p.blk_per_split < p.cols / 32 || (p.k_splits > 1) != (p.part != nullptr))
+    if (n < 1 || cols < 32 || cols % 32 != 0 || k_splits < 0 || !a16(x) || !a16(w) || !a16(xs) ||
+        (k_splits > 0 && (!part || !a16(part))))
         return hipErrorInvalidValue;
+    hipLaunchKernelGGL(norm_split_rows_kernel, dim3(n), dim3(kThreads), 0, s, x, part, k_splits,
+                       static_cast<long long>(n) * cols, w, cols, eps, xs);
+    return hipGetLastError();
+}
+
+hipError_t launch_product(int type, const ProductParams& p, hipStream_t s)
+{
+    const int n_blk = p.cols / 32, sub = (p.total_rows + 15) / 16, tiles = (p.n + 15) / 16, r = p.rows_per_group;
+    if (p.n < 1 || p.total_rows < 1 || p.cols < 64 || p.cols % 64 != 0 || (type == kQ6_K && p.cols % 256 != 0) ||
+        p.n_seg < 1 || p.n_seg > kGemvMaxSeg || p.row_bytes != static_cast<long long>(weight_row_bytes(type, p.cols)) ||
+        r < 1 || p.k_splits < 1 || p.blk_per_split < 2 || p.blk_per_split % 2 != 0 ||
+        static_cast<long long>(p.k_splits - 1) * p.blk_per_split >= n_blk ||
+        static_cast<long long>(p.k_splits) * p.blk_per_split < n_blk || (p.k_splits > 1) != (p.part != nullptr) ||
+        p.shares < 1)
+        return hipErrorInvalidValue;
+    if (p.pair && (p.n_seg != 2 || p.seg[0].rows != p.seg[1].rows || p.seg[0].rows % 32 != 0 || !p.hs ||
+                   p.kind == kProductTiled || p.k_splits > 1 || p.add))
+        return hipErrorInvalidValue;
+    const bool planes = p.planes || p.kind != kProductDirect;
+    if (planes ? !p.xs || !a16(p.xs) || p.norm_w : !p.x || !a16(p.x) || p.x_stride % 4 != 0) return hipErrorInvalidValue;
+    if (p.norm_w && (!a16(p.norm_w) || p.cols > kProductMaxNorm)) return hipErrorInvalidValue;
+    bool fits = false;
+    switch (p.kind) {
+    case kProductDirect:
+        fits = r <= direct_rows(type) && p.row_groups == (sub + r - 1) / r && p.n_tiles == tiles && p.k_splits == 1;
+        break;
+    case kProductResident:
+        fits = r <= resident_rows(type) && p.row_groups == (sub + r - 1) / r && p.n_tiles == tiles &&
+               p.shares <= tiles && p.blk_per_split <= kRangeBlocks;
+        break;
+    case kProductTiled:
+        fits = r <= 2 && p.row_groups == (p.total_rows + 64 * r - 1) / (64 * r) &&
+               p.n_tiles == (p.n + 16 * kTW - 1) / (16 * kTW) * kTW;
+        break;
+    }
+    if (!fits) return hipErrorInvalidValue;
     int rows = 0;
     for (int i = 0; i < p.n_seg; ++i) {
-        const uintptr_t align = type == kF32 || type == kF16 ? 16 : 2;
-        if (p.seg[i].rows < 1 || reinterpret_cast<uintptr_t>(p.seg[i].w) % align != 0) return hipErrorInvalidValue;
+        const uintptr_t align = type == kF32 || type == kF16 ? 16 : type == kQ6_K ? 2 : 4;
+        if (p.seg[i].rows < 1 || reinterpret_cast<uintptr_t>(p.seg[i].w) % align != 0 || (!p.seg[i].out && !p.pair))
+            return hipErrorInvalidValue;
         rows += p.seg[i].rows;
     }
     if (rows != p.total_rows) return hipErrorInvalidValue;
