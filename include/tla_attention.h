@@ -235,7 +235,7 @@ int tla_matmul(tla_engine* e, float* out_dev, const void* w_dev, const float* x_
  * 2048 columns are cut into ranges whose sums are added in order from a
  * second workspace.  Fewer vectors run as groups of matrix-vector products.
  * fp32 accumulation throughout: equal to the reference to fp32 rounding.
- * Used for the prompt's projections. */
+ * Used for the prompt's projections and a layer over several sequences. */
 int tla_matmul_batch(tla_engine* e, float* out_dev, const void* w_dev, const float* x_dev, int rows,
                      int cols, int n_tok, int type);
 
@@ -248,8 +248,10 @@ int tla_vec_add(tla_engine* e, float* out_dev, const float* x_dev, int size);
 
 /* The input half of the attention block for n_seq sequences
  * (src/forward.cpp:180-190): xb = rmsnorm(x, norm_w, eps) (skipped when
- * norm_w is NULL), q = Wq.xb, k = Wk.xb, v = Wv.xb, in one launch per 8
- * sequences (fewer when 8 x n_embd floats exceed 60 KiB).  x, q [n_seq][n_embd];
+ * norm_w is NULL), q = Wq.xb, k = Wk.xb, v = Wv.xb: one launch for one or two
+ * sequences, from 3 (F16 and F32 2, Q6_K 8; x and norm_w 16-byte aligned) the
+ * products of tla_matmul_batch, else one launch per 8 sequences (fewer when
+ * 8 x n_embd floats exceed 60 KiB).  x, q [n_seq][n_embd];
  * k, v [n_seq][kv_dim]; Wq [n_embd][n_embd],
  * Wk, Wv [kv_dim][n_embd], all of one type.  q and k leave unrotated, ready
  * for tla_decode with TLA_ROTATE (RoPE and the cache append are its
@@ -280,8 +282,9 @@ int tla_ffn_swiglu(tla_engine* e, float* out_dev, const float* in_dev, float* hb
                    const void* w_down_dev, int n_ff, int n_embd, int type);
 
 /* The FFN half of a layer (src/forward.cpp:215-228) for n_seq sequences:
- * x += ffn_swiglu(rmsnorm(x, norm_w, eps)), in two launches (rmsnorm + gate
- * and up projections; SiLU, gating, down projection and the residual add).
+ * x += ffn_swiglu(rmsnorm(x, norm_w, eps)): rmsnorm + gate and up
+ * projections, then SiLU, gating, down projection and the residual add (from
+ * 3 sequences, F16 and F32 2, Q6_K 8, as the products of tla_matmul_batch).
  * x [n_seq][n_embd]; hb_dev scratch [n_seq][2][n_ff] receives the raw gate
  * and up projections, except for one sequence of Q8_0 / Q4_0 / Q6_K weights
  * (n_embd <= 4096, n_ff even): then the gate half receives SiLU(gate) x up,

@@ -1,10 +1,12 @@
 """The split products of several tokens at the edges of their tiles, against
 fp64: the direct product (up to 16 tokens, or few rows), the resident one
 (more tokens; K in one or several ranges) and the tiled one (past 192
-tokens).
+tokens), and a layer's halves over several sequences, which run on them.
 
 Tolerance: a row is an fp32 sum of exact products in another order than the
-reference's, |gpu - fp64| <= 1e-5 sum |w x| (test_gpu_proj.py)."""
+reference's, |gpu - fp64| <= 1e-5 sum |w x| (test_gpu_proj.py).  A layer half
+that normalises first adds the norm's own rounding, a few 2^-24 of each x:
+2e-5; the FFN half chains three products: 8e-5 of the last one's sum."""
 import numpy as np
 import pytest
 
@@ -73,3 +75,42 @@ def test_product_infinities(W, engines, t, name, n, rows):
     assert np.isnan(got[2]).all()
     keep = [1] + list(range(3, n))
     rows_close(got[keep], raw, x[keep], t, rows, cols, 1e-5, f"{name} finite tokens")
+
+
+@pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("n", [3, 16, 17, 70, 200])
+def test_layer_halves(O, W, engines, t, name, n):
+    """tla_attn_qkv (with its rmsnorm), tla_attn_out and tla_ffn_block over n
+    sequences: the norm and SwiGLU fused where the shape allows, gate and up
+    left in hb as they were before."""
+    eng = engines(1, 64, 8, 2)
+    embd, kv, ff = 512, 128, 768
+    wq, wk, wv = (W.make_weights(t, r, embd, salt=i) for i, r in ((1, embd), (2, kv), (3, kv)))
+    wo = W.make_weights(t, embd, embd, salt=4)
+    wg, wu = W.make_weights(t, ff, embd, salt=5), W.make_weights(t, ff, embd, salt=6)
+    wd = W.make_weights(t, embd, ff, salt=7)
+    rg = np.random.default_rng(n)
+    x = rg.standard_normal((n, embd)).astype(np.float32)
+    nw = rg.uniform(0.5, 1.5, embd).astype(np.float32)
+    xn = np.stack([O.rmsnorm(r, nw, 1e-5) for r in x])
+    with device_arrays() as track:
+        d = {k: track(eng.array(v)) for k, v in
+             (("wq", wq), ("wk", wk), ("wv", wv), ("wo", wo), ("wg", wg), ("wu", wu), ("wd", wd), ("x", x), ("nw", nw))}
+        q, k, v = (track(eng.array((n, r))) for r in (embd, kv, kv))
+        eng.attn_qkv(n, q.ptr, k.ptr, v.ptr, d["x"].ptr, d["nw"].ptr, 1e-5, d["wq"].ptr, d["wk"].ptr, d["wv"].ptr, t)
+        for got, raw, rows in ((q, wq, embd), (k, wk, kv), (v, wv, kv)):
+            rows_close(got.download(), raw, xn, t, rows, embd, 2e-5, f"{name} qkv {rows} x {n}")
+        y = track(eng.array(x))
+        eng.attn_out(n, y.ptr, d["wo"].ptr, d["x"].ptr, t)
+        rows_close(y.download() - x, wo, x, t, embd, embd, 2e-5, f"{name} out x {n}")
+        hb = track(eng.array((n, 2, ff)))
+        eng.ffn_block(n, d["x"].ptr, d["nw"].ptr, 1e-5, d["wg"].ptr, d["wu"].ptr, d["wd"].ptr, ff, t, hb.ptr)
+        h, got = hb.download(), d["x"].download()
+    rows_close(h[:, 0], wg, xn, t, ff, embd, 2e-5, f"{name} gate x {n}")
+    rows_close(h[:, 1], wu, xn, t, ff, embd, 2e-5, f"{name} up x {n}")
+    g64, u64 = h[:, 0].astype(np.float64), h[:, 1].astype(np.float64)
+    act = g64 / (1 + np.exp(-g64)) * u64
+    w = Q.dequant(wd, t, embd, ff)
+    err = np.abs(got - (x + act @ w.T)) / (np.abs(act) @ np.abs(w).T + np.abs(x))
+    log(f"    {name} ffn x {n}: {err.max():.2e}")
+    assert err.max() <= 8e-5

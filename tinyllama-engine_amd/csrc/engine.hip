@@ -886,6 +886,15 @@ int tla_attn_qkv(tla_engine* e, int n_seq, float* q_dev, float* k_dev, float* v_
     if (reinterpret_cast<std::uintptr_t>(wk_dev) % 16 || reinterpret_cast<std::uintptr_t>(wv_dev) % 16)
         return fail(TLA_ERR_INVALID_ARGUMENT, "weights must be 16-byte aligned");
     if (int rc = set_device(e)) return rc;
+    if (batch_supported(type, embd, n_seq, x_dev, embd) && aligned16(norm_w_dev)) {
+        const GemvSegment segs[3] = {{static_cast<const unsigned char*>(wq_dev), q_dev, embd, embd},
+                                     {static_cast<const unsigned char*>(wk_dev), k_dev, kv, kv},
+                                     {static_cast<const unsigned char*>(wv_dev), v_dev, kv, kv}};
+        // without pending sums the norm only reads x
+        return norm_w_dev ? norm_product(e, type, segs, 3, embd, const_cast<float*>(x_dev), norm_w_dev, eps, n_seq, 0,
+                                         false)
+                          : matrix_batch(e, type, segs, 3, embd, x_dev, embd, n_seq, 0);
+    }
     for (int s0 = 0; s0 < n_seq; s0 += chunk) {
         const int nv = std::min(chunk, n_seq - s0);
         GemvParams p{};
@@ -916,6 +925,10 @@ int tla_attn_out(tla_engine* e, int n_seq, float* x_dev, const void* wo_dev, con
     const int chunk = gemv_chunk(n_seq, embd);
     if (int rc = check_gemv(type, embd, chunk, wo_dev)) return rc;
     if (int rc = set_device(e)) return rc;
+    if (batch_supported(type, embd, n_seq, xb2_dev, embd)) {
+        const GemvSegment seg{static_cast<const unsigned char*>(wo_dev), x_dev, embd, embd};
+        return matrix_batch(e, type, &seg, 1, embd, xb2_dev, embd, n_seq, 1);
+    }
     for (int s0 = 0; s0 < n_seq; s0 += chunk) {
         const int nv = std::min(chunk, n_seq - s0);
         GemvParams p{};
@@ -1619,6 +1632,10 @@ int tla_ffn_block(tla_engine* e, int n_seq, float* x_dev, const float* norm_w_de
     if (int rc = check_gemv(type, embd, chunk_up, w_up_dev)) return rc;
     if (int rc = check_gemv(type, n_ff, chunk_down, w_down_dev)) return rc;
     if (int rc = set_device(e)) return rc;
+    if (batch_supported(type, embd, n_seq, x_dev, embd) && n_ff % 64 == 0 &&
+        (type != kQ6_K || n_ff % 256 == 0) && aligned16(norm_w_dev) && aligned16(hb_dev))
+        return ffn_batch(e, type, x_dev, norm_w_dev, eps, w_gate_dev, w_up_dev, w_down_dev, n_ff, embd, n_seq, hb_dev,
+                         true, 0, nullptr);
     // hb_dev: [n_seq][2][n_ff], gate then up; for one sequence in a format
     // that pairs rows, the gate half receives SiLU(gate) x up directly.
     const bool paired = n_seq == 1 && gemv_can_pair(type, n_ff, embd);
