@@ -15,6 +15,7 @@
 
 
 #include "batch.h"
+#include "prefill.h"
 #include "tla_internal.h"
 
 using namespace tla;
@@ -132,6 +133,8 @@ struct tla_engine {
     size_t part_bytes = 0;
     unsigned char* kvp = nullptr; // prefill: K and V tiles as bf16 planes
     size_t kvp_bytes = 0;
+    float* pf_part = nullptr;     // its states of workgroups that share a query tile
+    int* pf_counters = nullptr;   // and their arrivals, zero between launches
     int* argmax_slot = nullptr;
     unsigned long long* amax_keys = nullptr;  // kAmaxSlots keys (tla_matmul_argmax)
     long long opt_split = 0;
@@ -264,6 +267,32 @@ int ensure_counters(tla_engine* e, size_t units)
     return TLA_OK;
 }
 
+// The fixed workspace of shared-out prefill launches (prefill.h).
+int ensure_prefill_part(tla_engine* e)
+{
+    if (e->pf_part) return TLA_OK;
+    const size_t states = static_cast<size_t>(kPrefillStates) * kPrefillStateBytes;
+    const size_t counters = kPrefillCounters * sizeof(int);
+    void* buf = nullptr;
+    TLA_HIP(hipMalloc(&buf, states + counters));
+    int* const cnt = reinterpret_cast<int*>(static_cast<char*>(buf) + states);
+    hipError_t rc = launch_zero(cnt, counters, e->stream);
+    if (rc == hipSuccess) rc = hipStreamSynchronize(e->stream);
+    if (rc != hipSuccess) {
+        (void)hipFree(buf);
+        TLA_HIP(rc);
+    }
+    e->pf_part = static_cast<float*>(buf);
+    e->pf_counters = cnt;
+    return TLA_OK;
+}
+
+// Whether [a, a + na) and [b, b + nb) floats share a byte.
+bool overlap(const float* a, long long na, const float* b, long long nb)
+{
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + 4 * static_cast<uintptr_t>(nb) && y < x + 4 * static_cast<uintptr_t>(na);
+}
 
 int check_engine(const tla_engine* e)
 {
@@ -435,6 +464,7 @@ int tla_engine_destroy(tla_engine* e)
     if (e->hs) (void)hipFree(e->hs);
     if (e->part) (void)hipFree(e->part);
     if (e->kvp) (void)hipFree(e->kvp);
+    if (e->pf_part) (void)hipFree(e->pf_part);
     if (e->argmax_slot) (void)hipFree(e->argmax_slot);
     if (e->amax_keys) (void)hipFree(e->amax_keys);
     if (e->rope) (void)hipFree(e->rope);
@@ -1196,6 +1226,24 @@ int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layer
     p.gqa = e->gqa;
     p.rotate = (flags & TLA_ROTATE) ? 1 : 0;
     p.scale_log2 = scale_log2(e->head_dim);
+    if (int rc = ensure_prefill_part(e)) return rc;
+    // One launch reads inputs and cache while it writes cache and output: a
+    // caller whose buffers overlap (k and v rows already in their place in the
+    // cache, say) keeps the two launches, where the rows are read before they
+    // are written.  (q and output may be the same rows.)
+    const long long n_in = static_cast<long long>(n_step_layers) * n_tok * e->kv_dim;
+    const long long n_out = n_in * e->gqa, n_cache = p.layer_stride * n_step_layers;
+    const float* const caches[2] = {key_cache_dev + p.layer_stride * layer0, value_cache_dev + p.layer_stride * layer0};
+    bool apart = true;
+    for (const float* in : {k_dev, v_dev}) {
+        apart &= !overlap(in, n_in, out_dev, n_out);
+        for (const float* cache : caches) apart &= !overlap(in, n_in, cache, n_cache);
+    }
+    for (const float* cache : caches)
+        apart &= !overlap(q_dev, n_out, cache, n_cache) && !overlap(out_dev, n_out, cache, n_cache);
+    if (apart && prefill_is_short(n_step_layers, c.n_head_kv, e->gqa, pos0, n_tok))
+        return launch(e, TLA_KERNEL_PREFILL, "prefill",
+                      [&] { return launch_prefill_short(p, e->pf_part, e->pf_counters, e->stream); });
     p.n_ptiles = (pos0 + n_tok + 31) / 32;
     if (int rc = ensure_buf(e, reinterpret_cast<void**>(&e->kvp), e->kvp_bytes,
                             prefill_planes_bytes(n_step_layers, c.n_head_kv, pos0, n_tok), "prefill K/V planes"))
@@ -1205,7 +1253,7 @@ int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layer
                         [&] { return launch_prefill_append(p, e->stream); }))
         return rc;
     if (int rc = launch(e, TLA_KERNEL_PREFILL, "prefill attention",
-                        [&] { return launch_prefill_attention(p, e->stream); }))
+                        [&] { return launch_prefill_attention(p, e->pf_part, e->pf_counters, e->stream); }))
         return rc;
     return ok();
 }
