@@ -226,7 +226,7 @@ int tla_matmul(tla_engine* e, float* out_dev, const void* w_dev, const float* x_
                int cols, int type);
 
 /* matmul() over a batch of n_tok vectors: out[t][rows] = W . x[t] (x
- * [n_tok][cols]).  From 3 vectors on (F16 and F32 from 2, Q6_K from 8) one
+ * [n_tok][cols]).  From 3 vectors on (F16 and F32 from 2, Q6_K from 6) one
  * split product: x split into three bf16 pieces, weights dequantised in
  * registers into exact bf16 pieces, every product of pieces exact in the fp32
  * accumulator of the bf16 matrix cores; up to 16 vectors, or for few rows,

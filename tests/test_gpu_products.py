@@ -16,11 +16,13 @@ from helpers import device_arrays, log
 pytestmark = pytest.mark.gpu
 
 TYPES = [(Q.F32, "f32"), (Q.F16, "f16"), (Q.Q4_0, "q4_0"), (Q.Q8_0, "q8_0"), (Q.Q6_K, "q6_k")]
-# direct: one token tile, remainders of rows and waves; resident: shares of
-# the tiles, K slices of 4 and 8 blocks, two K ranges with an uneven last one;
-# tiled: K ranges, token and row remainders
-SHAPES = [(17, 64, 3), (33, 320, 8), (4112, 256, 16), (9000, 512, 15), (4112, 1024, 17), (4200, 2048, 33),
-          (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250)]
+# direct: one token tile, remainders of rows and waves, groups of four blocks
+# that the row does not fill; resident: shares of the tiles, K slices of 4 and
+# 8 blocks, two K ranges with an uneven last one; tiled: K ranges, token and
+# row remainders
+SHAPES = [(17, 64, 3), (40, 192, 4), (4112, 1088, 2), (300, 3136, 4), (300, 3136, 5), (9000, 1344, 8),
+          (50, 2368, 3), (33, 256, 6), (33, 320, 8), (4112, 256, 16), (9000, 512, 15), (4112, 1024, 17),
+          (4200, 2048, 33), (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250)]
 
 
 def rows_close(got, raw, x, t, rows, cols, tol, what):

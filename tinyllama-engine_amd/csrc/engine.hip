@@ -689,10 +689,11 @@ int ensure_buf(tla_engine* e, void** buf, size_t& have, size_t bytes, const char
 
 // Fewest vectors that take the split products; fewer run as matrix-vector
 // launches (which read the weights once per 2 to 8 vectors).  Measured, TinyLlama's
-// matrices: Q4_0 / Q8_0 at 3 vectors 6.9-12.2 us against 7.9-18 us in the
+// matrices: Q4_0 / Q8_0 at 3 vectors 5.2-10.3 us against 7.9-18 us in the
 // matrix-vector launches (and at 2 those give a prompt's first layer the bits
-// of the token path); F16 / F32 at 2; Q6_K, whose decoding costs most, at 8.
-int min_batch(int type) { return type == kQ6_K ? 8 : type == kF16 || type == kF32 ? 2 : 3; }
+// of the token path); F16 / F32 at 2; Q6_K, whose decoding costs most, at 6
+// (32000 rows, 5 / 6 vectors: 54 / 54 us against 43 / 62).
+int min_batch(int type) { return type == kQ6_K ? 6 : type == kF16 || type == kF32 ? 2 : 3; }
 
 bool aligned16(const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; }
 

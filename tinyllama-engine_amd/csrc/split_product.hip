@@ -562,15 +562,24 @@ __device__ __forceinline__ void store_gated(const ProductParams& p, float sum, i
 // from zero): one token tile does not repay splitting both operands (2560 x
 // 2048, 3 tokens, 9.2 us split, 8.4 so; F16 with three row subtiles 12.9
 // split, 15.1 so).
+//
+// Up to 16 / kShare tokens leave rows of the x operand free: its row set u (of
+// kShare) holds the tokens in block u of kShare consecutive ones, so that one
+// load and split of x serves them all.  Block u's products go into accumulators
+// of their own, of which only row set u counts; the sets meet with the waves'
+// sums.  4 tokens, kShare 1 / 2 / 4: F16, 2048 x 5632 13.6 / 11.0 / 10.5 us;
+// Q8_0, 2048 x 5632 12.3 / 9.7 / 8.9, 2560 x 2048 6.6 / 5.7 / 5.5.  (More blocks in
+// flight instead, 12 or 16: F16, 2048 x 5632, 13.2 -> 14.4 and 16.2.)
 enum XSource { kXRows, kXNormRows, kXPlanes };
 
-template <int kType, int kR, int kSrc, int kDepth>
+template <int kType, int kR, int kSrc, int kDepth, int kShare>
 __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const ProductParams p)
 {
     constexpr int kN = Fmt<kType>::kN;
     constexpr bool kNorm = kSrc == kXNormRows;
     constexpr bool kFp32 = kSrc != kXPlanes && kType == kF32;
     constexpr int kCombos = 4 * kR;
+    constexpr int kTok = 16 / kShare;  // tokens per tile row set
     __shared__ float s_red[kWaves][kCombos][64];
     __shared__ float s_ss[kWaves][16];
     __shared__ __align__(16) float s_norm[kNorm ? kProductMaxNorm : 4];
@@ -578,32 +587,37 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
     const int j = lane & 15, g = lane >> 4;
     const int n_blk = p.cols >> 5, tile = blockIdx.y;
     const int sub0 = blockIdx.x * kR;
-    // blocks wave + kWaves i, i < nb
-    const int nb = wave < n_blk ? (n_blk - wave + kWaves - 1) / kWaves : 0;
+    // groups of kShare blocks: wave + kWaves i, i < nb
+    const int n_grp = (n_blk + kShare - 1) / kShare;
+    const int nb = wave < n_grp ? (n_grp - wave + kWaves - 1) / kWaves : 0;
+    const int jt = j % kTok, jb = j / kTok;  // this lane's token, and its block of a group
     const unsigned char* wrow[kR];
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
         const TileRow rs = tile_row(p, sub0 + r, j);
         wrow[r] = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
     }
-    const float* const xrow = p.x + static_cast<long long>(min(16 * tile + j, p.n - 1)) * p.x_stride + 8 * g;
+    const float* const xrow = p.x + static_cast<long long>(min(16 * tile + jt, p.n - 1)) * p.x_stride + 8 * g;
 
     struct Stage {
-        WRaw<kType> w[kR];
+        WRaw<kType> w[kShare][kR];
         u32x4 x[kSrc == kXPlanes ? 3 : 2];  // eight floats, or their planes
     } st[kDepth];
     // (past the wave's last block that one again, never used: no load sits
     // behind a branch, where the compiler would wait for all in flight)
     const auto load = [&](Stage& t, int i) __attribute__((always_inline)) {
-        const int kb = min(wave + kWaves * min(i, max(nb - 1, 0)), n_blk - 1);
+        const int kb = kShare * min(wave + kWaves * min(i, max(nb - 1, 0)), n_grp - 1);
+        const int xb = min(kb + jb, n_blk - 1);
         const unsigned char* const src =
-            kSrc == kXPlanes ? p.xs + plane_chunk(tile, kb, 0, n_blk) + 16 * lane
-                             : reinterpret_cast<const unsigned char*>(xrow + 32 * kb);
+            kSrc == kXPlanes ? p.xs + plane_chunk(tile, xb, 0, n_blk) + 16 * (16 * g + jt)
+                             : reinterpret_cast<const unsigned char*>(xrow + 32 * xb);
 #pragma unroll
         for (int i2 = 0; i2 < (kSrc == kXPlanes ? 3 : 2); ++i2)
             t.x[i2] = *reinterpret_cast<const u32x4*>(src + (kSrc == kXPlanes ? 1024 : 16) * i2);
 #pragma unroll
-        for (int r = 0; r < kR; ++r) load_w<kType>(t.w[r], wrow[r], kb, g);
+        for (int u = 0; u < kShare; ++u)
+#pragma unroll
+            for (int r = 0; r < kR; ++r) load_w<kType>(t.w[u][r], wrow[r], min(kb + u, n_blk - 1), g);
     };
 #pragma unroll
     for (int d = 0; d < kDepth; ++d) {
@@ -618,51 +632,61 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     }
-    floatx4 acc[kR];
+    floatx4 acc[kShare][kR];
 #pragma unroll
-    for (int r = 0; r < kR; ++r) acc[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < kShare; ++u)
+#pragma unroll
+        for (int r = 0; r < kR; ++r) acc[u][r] = floatx4{0.f, 0.f, 0.f, 0.f};
     float ss = 0.f;
     const auto block = [&](const Stage& t, int i) __attribute__((always_inline)) {
-        const int kb = wave + kWaves * i;
+        const int kb = kShare * (wave + kWaves * i);
+        const bool in = kShare == 1 || kb + jb < n_blk;  // a block past the row adds zeros
         split_f32x8 v;
         if constexpr (kSrc != kXPlanes) {
             const float4 xa = __builtin_bit_cast(float4, t.x[0]), xb = __builtin_bit_cast(float4, t.x[1]);
             v = split_f32x8{xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
+            if (kShare > 1) v = in ? v : split_f32x8{};
             if constexpr (kNorm) {
-                const float4* const nw = reinterpret_cast<const float4*>(s_norm + 32 * kb + 8 * g);
+                const float4* const nw = reinterpret_cast<const float4*>(s_norm + 32 * (kShare == 1 ? kb : min(kb + jb, n_blk - 1)) + 8 * g);
                 const float4 na = nw[0], nb4 = nw[1];
-                ss += sum_sq4(xa) + sum_sq4(xb);
+                ss += kShare == 1 || in ? sum_sq4(xa) + sum_sq4(xb) : 0.f;
                 v *= split_f32x8{na.x, na.y, na.z, na.w, nb4.x, nb4.y, nb4.z, nb4.w};
             }
         }
         if constexpr (kFp32) {
-            floatx4 sum[kR];
-            split_f32x8 w[kR];
 #pragma unroll
-            for (int r = 0; r < kR; ++r) {
-                sum[r] = floatx4{0.f, 0.f, 0.f, 0.f};
-                w[r] = float_w<kType>(t.w[r]);
+            for (int u = 0; u < kShare; ++u) {
+                floatx4 sum[kR];
+                split_f32x8 w[kR];
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    sum[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    w[r] = float_w<kType>(t.w[u][r]);
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int r = 0; r < kR; ++r)
+                        sum[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], w[r][e], sum[r], 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < kR; ++r) acc[u][r] += sum[r];
             }
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-#pragma unroll
-                for (int r = 0; r < kR; ++r)
-                    sum[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e], w[r][e], sum[r], 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < kR; ++r) acc[r] += sum[r];
         } else {
             bf16x8 x[3];
             if constexpr (kSrc == kXPlanes) {
 #pragma unroll
-                for (int pl = 0; pl < 3; ++pl) x[pl] = __builtin_bit_cast(bf16x8, t.x[pl]);
+                for (int pl = 0; pl < 3; ++pl) x[pl] = in ? __builtin_bit_cast(bf16x8, t.x[pl]) : bf16x8{};
             } else {
                 split3x8(v, x[0], x[1], x[2]);
             }
-            bf16x8 b[kR][kN];
-            unsigned d[kR];
 #pragma unroll
-            for (int r = 0; r < kR; ++r) decode_w<kType>(t.w[r], kb, g, b[r], d[r]);
-            block_products<kType, kR>(x, b, d, acc);
+            for (int u = 0; u < kShare; ++u) {
+                bf16x8 b[kR][kN];
+                unsigned d[kR];
+#pragma unroll
+                for (int r = 0; r < kR; ++r) decode_w<kType>(t.w[u][r], min(kb + u, n_blk - 1), g, b[r], d[r]);
+                block_products<kType, kR>(x, b, d, acc[u]);
+            }
         }
     };
     int i0 = 0;
@@ -681,7 +705,13 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
 #pragma unroll
     for (int r = 0; r < kR; ++r)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s_red[wave][4 * r + q][lane] = acc[r][q];
+        for (int q = 0; q < 4; ++q) {
+            // the set of block g kShare / 4 has its tokens in this lane group's rows
+            float sum = acc[0][r][q];
+#pragma unroll
+            for (int u = 1; u < kShare; ++u) sum = g * kShare / 4 == u ? acc[u][r][q] : sum;
+            s_red[wave][4 * r + q][lane] = sum;
+        }
     if constexpr (kNorm) {
         ss += __shfl_xor(ss, 16);
         ss += __shfl_xor(ss, 32);
@@ -693,9 +723,11 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
     for (int c0 = 0; c0 < kCombos; c0 += kWaves) {
         const int c = c0 + wave, t = 16 * tile + 4 * g + (c & 3);
         if (c >= kCombos) return;
-        float sum = s_red[0][c][lane];
+        float sum = 0.f;
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) sum += s_red[w][c][lane];
+        for (int u = 0; u < kShare; ++u)
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) sum += s_red[w][c][(lane + 64 / kShare * u) & 63];
         const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
         const bool ok = rs.ok && t < p.n;
         if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
@@ -706,9 +738,11 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
             });
         }
         if constexpr (kNorm) {
-            float s2 = s_ss[0][4 * g + (c & 3)];
+            float s2 = 0.f;
 #pragma unroll
-            for (int w = 1; w < kWaves; ++w) s2 += s_ss[w][4 * g + (c & 3)];
+            for (int u = 0; u < kShare; ++u)
+#pragma unroll
+                for (int w = 0; w < kWaves; ++w) s2 += s_ss[w][(4 * g + (c & 3) + kTok * u) & 15];
             sum *= 1.0f / sqrtf(s2 / static_cast<float>(p.cols) + p.eps);
         }
         if (ok && rs.out) {
@@ -1075,32 +1109,54 @@ __global__ __launch_bounds__(kThreads) void range_sum_kernel(const ProductParams
 constexpr int direct_rows(int type) { return type == kQ6_K ? 2 : kMaxRows; }
 constexpr int resident_rows(int type) { return type == kF32 ? 1 : type == kF16 || type == kQ6_K ? 2 : kMaxRows; }
 
-template <int kType, int kR, int kDepth>
+template <int kType, int kR, int kDepth, int kShare>
 hipError_t launch_direct_depth(const ProductParams& p, hipStream_t s)
 {
     const dim3 grid(static_cast<unsigned>(p.row_groups), static_cast<unsigned>(p.n_tiles)), block(kWaves * 64);
     if (p.planes)
-        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXPlanes, kDepth>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXPlanes, kDepth, kShare>), grid, block, 0, s, p);
     else if (p.norm_w)
-        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXNormRows, kDepth>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXNormRows, kDepth, kShare>), grid, block, 0, s, p);
     else
-        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXRows, kDepth>), grid, block, 0, s, p);
+        hipLaunchKernelGGL((direct_product_kernel<kType, kR, kXRows, kDepth, kShare>), grid, block, 0, s, p);
     return hipGetLastError();
 }
 
 // Blocks in flight per wave: all of 2048 columns with one row subtile (fewer
 // where the row has fewer: a load past the end is made, not used), else four,
 // which is what the registers hold beside three subtiles.
+template <int kType, int kR, int kShare>
+hipError_t launch_direct_share(const ProductParams& p, hipStream_t s)
+{
+    if constexpr (kR == 1) {
+        const int groups = (p.cols / 32 + kShare * kWaves - 1) / (kShare * kWaves);
+        if constexpr (kShare == 4)
+            return launch_direct_depth<kType, 1, 2, 4>(p, s);
+        else if constexpr (kShare == 2)
+            return groups <= 1   ? launch_direct_depth<kType, 1, 1, 2>(p, s)
+                   : groups <= 2 ? launch_direct_depth<kType, 1, 2, 2>(p, s)
+                                 : launch_direct_depth<kType, 1, 4, 2>(p, s);
+        else
+            return groups <= 2   ? launch_direct_depth<kType, 1, 2, 1>(p, s)
+                   : groups <= 4 ? launch_direct_depth<kType, 1, 4, 1>(p, s)
+                                 : launch_direct_depth<kType, 1, 8, 1>(p, s);
+    } else {
+        return launch_direct_depth<kType, kR, kShare == 1 ? 4 : 2, kShare>(p, s);
+    }
+}
+
+// Up to 8 tokens two blocks share an x operand, up to 4 tokens four: with one
+// row subtile (the accumulators of four for three subtiles leave no registers
+// for loads: F32, 11264 x 2048, 3 tokens 28 against 18 us; Q4_0, 32000 rows, 26
+// against 22) and more than one group of them per wave (900 x 1024, F16 4.5
+// against 4.3 us).
 template <int kType, int kR>
 hipError_t launch_direct(const ProductParams& p, hipStream_t s)
 {
-    if constexpr (kR == 1) {
-        const int blocks = (p.cols / 32 + kWaves - 1) / kWaves;
-        return blocks <= 2   ? launch_direct_depth<kType, 1, 2>(p, s)
-               : blocks <= 4 ? launch_direct_depth<kType, 1, 4>(p, s)
-                             : launch_direct_depth<kType, 1, 8>(p, s);
-    } else if constexpr (kR <= direct_rows(kType)) {
-        return launch_direct_depth<kType, kR, 4>(p, s);
+    if constexpr (kR <= direct_rows(kType)) {
+        if constexpr (kR == 1)
+            if (p.n <= 4 && p.cols / 32 > 4 * kWaves) return launch_direct_share<kType, kR, 4>(p, s);
+        return p.n <= 8 ? launch_direct_share<kType, kR, 2>(p, s) : launch_direct_share<kType, kR, 1>(p, s);
     } else {
         return hipErrorInvalidValue;
     }
