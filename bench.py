@@ -79,7 +79,7 @@ def log(msg):
 # digest, and its byte count is used only while the sources are unchanged.
 KERNEL_SOURCES = {
     "decode_split_kernel": ("decode.hip", "tla_internal.h", "rope_math.h", "lane_math.h"),
-    "prefill_attention_kernel": ("prefill.hip", "tla_internal.h", "rope_math.h", "lane_math.h", "bf16_split.h"),
+    "prefill_attention_kernel": ("prefill.hip", "prefill.h", "tla_internal.h", "rope_math.h", "lane_math.h", "bf16_split.h"),
     "gemv_kernel": ("gemv.hip", "tla_internal.h", "row_math.h", "rope_math.h"),
 }
 

@@ -465,16 +465,16 @@ __device__ __forceinline__ split_f32x8 float_w(const WRaw<kType>& w)
 // One block's products for kR row subtiles: acc (+)= the products of pieces
 // (x_p, b_i) with i + p <= 2, smallest terms first, scaled by the block scale
 // (the bits of a half) where there is one.  Each block is summed from zero:
-// carried through the matrix cores from block to block, F16 sums were 2.2e-7
-// off fp64 at 2048 columns against 1e-7.
-template <int kType, int kR>
+// carried through the matrix cores from block to block (kCarry), F16 sums were
+// 2.2e-7 off fp64 at 2048 columns against 1e-7.
+template <int kType, int kR, bool kCarry = false>
 __device__ __forceinline__ void block_products(const bf16x8 (&x)[3], const bf16x8 (&b)[kR][Fmt<kType>::kN],
                                                const unsigned (&d)[kR], floatx4 (&acc)[kR])
 {
     constexpr int kN = Fmt<kType>::kN;
     floatx4 t[kR];
 #pragma unroll
-    for (int r = 0; r < kR; ++r) t[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < kR; ++r) t[r] = kCarry ? acc[r] : floatx4{0.f, 0.f, 0.f, 0.f};
     if constexpr (kN >= 3) {
 #pragma unroll
         for (int r = 0; r < kR; ++r) t[r] = mfma(x[0], b[r][kN - 1], t[r]);
@@ -495,6 +495,8 @@ __device__ __forceinline__ void block_products(const bf16x8 (&x)[3], const bf16x
             const float s = half_to_float(d[r]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) acc[r][q] = fmaf(s, t[r][q], acc[r][q]);
+        } else if constexpr (kCarry) {
+            acc[r] = t[r];
         } else {
             acc[r] += t[r];
         }
@@ -920,7 +922,9 @@ __global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const Pro
 // ahead.  Bound by its barrier per block and LDS reads; kept where the
 // resident product holds too few rows or needs several K ranges (512 tokens,
 // us, tiled / resident: F16 11264 x 2048 105 / 123, F32 155 / 191, Q8_0
-// 2048 x 5632 61 / 69; at 160 tokens 57 / 55, 82 / 76, 35 / 33).
+// 2048 x 5632 61 / 69; 100 tokens F16 11264 x 2048 42 / 45, F32 2048 x 5632
+// 35 / 46, F32 2560 x 2048 25 / 23).  Types without a scale carry their sums
+// through the matrix cores (64 tokens' adds a block cost F16 6 %).
 template <int kType, int kRW>
 __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const ProductParams p)
 {
@@ -940,6 +944,7 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
     const int n_blk = p.cols >> 5;
     const int row0 = (tx * kTileWaves + wave) * 16 * kRW;
     const int s0 = ty * kTW;  // first token subtile
+    const int live = min(kTW, (p.n + 15) / 16 - s0);  // subtiles with tokens
     // K range of this workgroup: blocks [kb_lo, kb_hi) (grid z splits K)
     const int kb_lo = tz * p.blk_per_split;
     const int kb_hi = min(kb_lo + p.blk_per_split, n_blk);
@@ -1028,8 +1033,7 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
             unsigned d[kRW];
 #pragma unroll
             for (int r = 0; r < kRW; ++r) decode_w<kType>(wr_this[r], kb, g, b[r], d[r]);
-#pragma unroll
-            for (int s = 0; s < kTW; ++s) {
+            const auto token_tile = [&](int s) __attribute__((always_inline)) {
                 bf16x8 a[3];
 #pragma unroll
                 for (int pl = 0; pl < 3; ++pl)
@@ -1037,10 +1041,19 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
 #pragma unroll
                 for (int r = 0; r < kRW; ++r) {
                     floatx4 one[1] = {acc[r][s]};
-                    block_products<kType, 1>(a, reinterpret_cast<const bf16x8(&)[1][Fmt<kType>::kN]>(b[r]),
-                                             reinterpret_cast<const unsigned(&)[1]>(d[r]), one);
+                    block_products<kType, 1, !Fmt<kType>::kScaled>(
+                        a, reinterpret_cast<const bf16x8(&)[1][Fmt<kType>::kN]>(b[r]),
+                        reinterpret_cast<const unsigned(&)[1]>(d[r]), one);
                     acc[r][s] = one[0];
                 }
+            };
+            if (live == kTW) {
+#pragma unroll
+                for (int s = 0; s < kTW; ++s) token_tile(s);
+            } else {
+#pragma unroll
+                for (int s = 0; s < kTW - 1; ++s)
+                    if (s < live) token_tile(s);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1230,7 +1243,11 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         return;
     }
     const int ranges = (n_blk + kRangeBlocks - 1) / kRangeBlocks;
-    const bool tiled = p->n > 192 && type != kQ6_K && !p->pair &&
+    const int tiled_past = type == kF16   ? 80
+                           : type != kF32 ? 160
+                           : ranges > 1   ? 64
+                                          : p->total_rows > 4096 ? 80 : 112;
+    const bool tiled = p->n > tiled_past && type != kQ6_K && !p->pair &&
                        (ranges > 1 || (type == kF16 && p->total_rows > 4096) || (type == kF32 && p->total_rows > 2048));
     int splits = std::max(ranges, std::min(opt_k, n_blk / 2));
     if (tiled) {
