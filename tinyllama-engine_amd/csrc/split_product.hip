@@ -465,16 +465,16 @@ __device__ __forceinline__ split_f32x8 float_w(const WRaw<kType>& w)
 // One block's products for kR row subtiles: acc (+)= the products of pieces
 // (x_p, b_i) with i + p <= 2, smallest terms first, scaled by the block scale
 // (the bits of a half) where there is one.  Each block is summed from zero:
-// carried through the matrix cores from block to block (kCarry), F16 sums were
-// 2.2e-7 off fp64 at 2048 columns against 1e-7.
-template <int kType, int kR, bool kCarry = false>
+// carried through the matrix cores from block to block, F16 sums were 2.2e-7
+// off fp64 at 2048 columns against 1e-7.
+template <int kType, int kR>
 __device__ __forceinline__ void block_products(const bf16x8 (&x)[3], const bf16x8 (&b)[kR][Fmt<kType>::kN],
                                                const unsigned (&d)[kR], floatx4 (&acc)[kR])
 {
     constexpr int kN = Fmt<kType>::kN;
     floatx4 t[kR];
 #pragma unroll
-    for (int r = 0; r < kR; ++r) t[r] = kCarry ? acc[r] : floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < kR; ++r) t[r] = floatx4{0.f, 0.f, 0.f, 0.f};
     if constexpr (kN >= 3) {
 #pragma unroll
         for (int r = 0; r < kR; ++r) t[r] = mfma(x[0], b[r][kN - 1], t[r]);
@@ -495,8 +495,6 @@ __device__ __forceinline__ void block_products(const bf16x8 (&x)[3], const bf16x
             const float s = half_to_float(d[r]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) acc[r][q] = fmaf(s, t[r][q], acc[r][q]);
-        } else if constexpr (kCarry) {
-            acc[r] = t[r];
         } else {
             acc[r] += t[r];
         }
@@ -923,8 +921,9 @@ __global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const Pro
 // resident product holds too few rows or needs several K ranges (512 tokens,
 // us, tiled / resident: F16 11264 x 2048 105 / 123, F32 155 / 191, Q8_0
 // 2048 x 5632 61 / 69; 100 tokens F16 11264 x 2048 42 / 45, F32 2048 x 5632
-// 35 / 46, F32 2560 x 2048 25 / 23).  Types without a scale carry their sums
-// through the matrix cores (64 tokens' adds a block cost F16 6 %).
+// 35 / 46, F32 2560 x 2048 25 / 23).  Carrying the sums
+// of types without a scale through the matrix cores was 3-6 % faster and put a
+// layer of F16 over 100 sequences 3.6e-7 off fp64 against 1.4e-7.
 template <int kType, int kRW>
 __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const ProductParams p)
 {
@@ -1041,7 +1040,7 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
 #pragma unroll
                 for (int r = 0; r < kRW; ++r) {
                     floatx4 one[1] = {acc[r][s]};
-                    block_products<kType, 1, !Fmt<kType>::kScaled>(
+                    block_products<kType, 1>(
                         a, reinterpret_cast<const bf16x8(&)[1][Fmt<kType>::kN]>(b[r]),
                         reinterpret_cast<const unsigned(&)[1]>(d[r]), one);
                     acc[r][s] = one[0];
