@@ -60,8 +60,18 @@ def test_product_infinities(W, engines, t, name, n, rows):
     """A token with an infinity, one with the largest float and one with a NaN
     give what fp32 products give (the bf16 pieces of an infinity alone would
     cancel to NaN); the other tokens are untouched by them."""
-    eng = engines(1, 64)
-    cols = 256
+    infinities(W, engines(1, 64), t, name, n, rows, 256)
+
+
+# where the tiled product runs: F16 and F32 in one K range, every format but
+# Q6_K (which keeps the resident one) in several
+@pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("n,rows,cols", [(130, 4128, 256), (170, 72, 2304)])
+def test_product_infinities_many_tokens(W, engines, t, name, n, rows, cols):
+    infinities(W, engines(1, 64), t, name, n, rows, cols)
+
+
+def infinities(W, eng, t, name, n, rows, cols):
     raw = W.make_weights(t, rows, cols, salt=3)
     x = np.random.default_rng(5).standard_normal((n, cols)).astype(np.float32)
     x[0, 40], x[1, 7], x[2, 200] = np.inf, np.finfo(np.float32).max, np.nan
