@@ -90,6 +90,33 @@ def infinities(W, eng, t, name, n, rows, cols):
 
 
 @pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("n", [8, 40])
+def test_norm_of_huge_rows(O, W, engines, t, name, n):
+    """A finite row whose sum of squares overflows is scaled by zero, as the
+    reference's rmsnorm does (the product itself of such a row passes the
+    largest float: taken over the unscaled row and multiplied by zero after, it
+    would be NaN); a row with an infinity is NaN; the others stay."""
+    eng = engines(1, 64, 8, 2)
+    embd, kv = 512, 128
+    wq, wk, wv = (W.make_weights(t, r, embd, salt=i) for i, r in ((1, embd), (2, kv), (3, kv)))
+    x = np.random.default_rng(6).standard_normal((n, embd)).astype(np.float32)
+    nw = np.random.default_rng(7).uniform(0.5, 1.5, embd).astype(np.float32)
+    x[0] = np.copysign(np.float32(3e38), x[0])
+    x[1, 300] = -np.inf
+    with np.errstate(all="ignore"):
+        xn = np.stack([O.rmsnorm(r, nw, 1e-5) for r in x])
+    assert not xn[0].any() and np.isnan(xn[1, 300])
+    with device_arrays() as track:
+        d = [track(eng.array(a)) for a in (wq, wk, wv, x, nw)]
+        q, k, v = (track(eng.array((n, r))) for r in (embd, kv, kv))
+        eng.attn_qkv(n, q.ptr, k.ptr, v.ptr, d[3].ptr, d[4].ptr, 1e-5, d[0].ptr, d[1].ptr, d[2].ptr, t)
+        for got, raw, rows in ((q.download(), wq, embd), (k.download(), wk, kv), (v.download(), wv, kv)):
+            assert not got[0].any()
+            assert np.isnan(got[1]).all()
+            rows_close(got[2:], raw, xn[2:], t, rows, embd, 2e-5, f"{name} qkv {rows} x {n}")
+
+
+@pytest.mark.parametrize("t,name", TYPES)
 @pytest.mark.parametrize("n", [3, 16, 17, 70, 200])
 def test_layer_halves(O, W, engines, t, name, n):
     """tla_attn_qkv (with its rmsnorm), tla_attn_out and tla_ffn_block over n

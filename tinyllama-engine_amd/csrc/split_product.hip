@@ -730,20 +730,24 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
             for (int w = 0; w < kWaves; ++w) sum += s_red[w][c][(lane + 64 / kShare * u) & 63];
         const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
         const bool ok = rs.ok && t < p.n;
-        if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
-            const unsigned char* const wr = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
-            const float* const xr = p.x + t * p.x_stride;
-            sum = plain_sum<kType>(wr, 0, p.cols, [&](int col) {
-                return kSrc == kXPlanes ? plane_value(p.xs, t, col, n_blk) : kNorm ? xr[col] * s_norm[col] : xr[col];
-            });
-        }
+        float rms = 1.f;
         if constexpr (kNorm) {
             float s2 = 0.f;
 #pragma unroll
             for (int u = 0; u < kShare; ++u)
 #pragma unroll
                 for (int w = 0; w < kWaves; ++w) s2 += s_ss[w][(4 * g + (c & 3) + kTok * u) & 15];
-            sum *= 1.0f / sqrtf(s2 / static_cast<float>(p.cols) + p.eps);
+            rms = 1.0f / sqrtf(s2 / static_cast<float>(p.cols) + p.eps);
+        }
+        if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
+            // (normalised value by value: 1 / rms may be zero for a finite row)
+            const unsigned char* const wr = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
+            const float* const xr = p.x + t * p.x_stride;
+            sum = plain_sum<kType>(wr, 0, p.cols, [&](int col) {
+                return kSrc == kXPlanes ? plane_value(p.xs, t, col, n_blk) : kNorm ? xr[col] * rms * s_norm[col] : xr[col];
+            });
+        } else if constexpr (kNorm) {
+            sum *= rms;
         }
         if (ok && rs.out) {
             float* const o = rs.out + rs.row + t * rs.stride;
