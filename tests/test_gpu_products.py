@@ -71,6 +71,31 @@ def test_product_infinities_many_tokens(W, engines, t, name, n, rows, cols):
     infinities(W, engines(1, 64), t, name, n, rows, cols)
 
 
+@pytest.mark.parametrize("n,rows,cols", [(12, 2048, 5632), (512, 11264, 2048)])
+def test_nan_token_costs_little(W, engines, n, rows, cols):
+    """A token with a NaN does not hold up the batch it is in: the product stays
+    under three times its time without (1.1 to 1.5 times measured; 10 and 35
+    times where a lane walked over the columns for each of the token's sums)."""
+    eng = engines(1, 64)
+    x = np.random.default_rng(9).standard_normal((n, cols)).astype(np.float32)
+    best = []
+    with device_arrays() as track:
+        w, out, xd = track(eng.array(W.make_weights(Q.Q8_0, rows, cols, salt=3))), track(eng.array((n, rows))), track(eng.array(x))
+        for value in (0.5, np.nan):
+            x[5, 77] = value
+            xd.upload(x)
+            times = []
+            for _ in range(6):
+                eng.event(0)
+                for _ in range(5):
+                    eng.matmul_batch(out.ptr, w.ptr, xd.ptr, rows, cols, n, Q.Q8_0)
+                eng.event(1)
+                times.append(eng.elapsed(0, 1))
+            best.append(min(times))
+    log(f"    {best[0] * 200:.1f} us, with a NaN {best[1] * 200:.1f} us")
+    assert best[1] < 3 * best[0]
+
+
 def infinities(W, eng, t, name, n, rows, cols):
     raw = W.make_weights(t, rows, cols, salt=3)
     x = np.random.default_rng(5).standard_normal((n, cols)).astype(np.float32)

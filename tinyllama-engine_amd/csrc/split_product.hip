@@ -401,19 +401,6 @@ __device__ __forceinline__ float weight_at(const unsigned char* wrow, int c)
     }
 }
 
-// Pieces of an infinite operand can cancel to a NaN (inf - inf, 0 * inf), and a
-// block's unscaled sum can pass the largest float, where the products
-// themselves do neither: a sum that is not finite is taken again in plain
-// fp32 over columns [c0, c1), x from its row or from the planes.
-template <int kType, class X>
-__device__ __forceinline__ float plain_sum(const unsigned char* wrow, int c0, int c1, X&& x_at)
-{
-    float s = 0.f;
-#pragma unroll 1
-    for (int c = c0; c < c1; ++c) s += weight_at<kType>(wrow, c) * x_at(c);
-    return s;
-}
-
 __device__ __forceinline__ float plane_value(const unsigned char* xs, int t, int c, int n_blk)
 {
     float v = 0.f;
@@ -422,6 +409,64 @@ __device__ __forceinline__ float plane_value(const unsigned char* xs, int t, int
         v += static_cast<float>(*reinterpret_cast<const __bf16*>(
             xs + plane_chunk(t >> 4, c >> 5, pl, n_blk) + 16 * (16 * (c >> 3 & 3) + (t & 15)) + 2 * (c & 7)));
     return v;
+}
+
+// Pieces of an infinite operand can cancel to a NaN (inf - inf, 0 * inf), and a
+// block's unscaled sum can pass the largest float, where the products
+// themselves do neither: a sum that is not finite (redo) is taken again in plain
+// fp32 over columns [c0, c1), multiples of 32, of weight row wrow and token t,
+// x_at(t, c, scale) from its row or from the planes; bad8(c8): whether the eight
+// columns 8 c8 .. of the lane's own token make every sum NaN.  All lanes of the
+// wave call it, the sixteen of a group with one t: they share the search for
+// NaNs, and the wave takes the other sums one after another, all lanes on each.
+// (One token of 512 with a NaN / an infinity, Q4_0, 11264 x 2048, 103 us without:
+// a lane per sum 1110 / 1110 us; so 109 / 341.)
+template <int kType, class B, class X>
+__device__ __forceinline__ float taken_again(float sum, bool redo, const unsigned char* wrow, int t, float scale,
+                                             int c0, int c1, B&& bad8, X&& x_at)
+{
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // nothing of this is computed ahead, in registers the loops need
+    bool bad = false;
+#pragma unroll 1
+    for (int c8 = c0 / 8 + (lane & 15); c8 < c1 / 8; c8 += 16) bad |= bad8(c8);
+    bad = (__ballot(bad) >> (lane & 48) & 0xFFFF) != 0;
+    if (redo && bad) sum = __builtin_nanf("");
+    const unsigned long long row = reinterpret_cast<unsigned long long>(wrow);
+#pragma unroll 1
+    for (unsigned long long left = __ballot(redo && !bad); left; left &= left - 1) {
+        const int from = __builtin_ctzll(left);
+        const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(row), from);
+        const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(row >> 32), from);
+        const unsigned char* const w = reinterpret_cast<const unsigned char*>(static_cast<unsigned long long>(hi) << 32 | lo);
+        const int tok = __builtin_amdgcn_readlane(t, from);
+        const float sc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, scale), from));
+        float s = 0.f;
+#pragma unroll 1
+        for (int c = c0 + lane; c < c1; c += 64) s += weight_at<kType>(w, c) * x_at(tok, c, sc);
+#pragma unroll
+        for (int d = 32; d; d >>= 1) s += __shfl_xor(s, d);
+        sum = lane == from ? s : sum;
+    }
+    return sum;
+}
+
+// The same for x in the planes.
+template <int kType>
+__device__ __forceinline__ float taken_again(float sum, bool redo, const unsigned char* wrow, int t, int c0, int c1,
+                                             const unsigned char* xs, int n_blk)
+{
+    return taken_again<kType>(
+        sum, redo, wrow, t, 1.f, c0, c1,
+        [&](int c8) {
+            const bf16x8 x0 = *reinterpret_cast<const bf16x8*>(xs + plane_chunk(t >> 4, c8 >> 2, 0, n_blk) +
+                                                               16 * (16 * (c8 & 3) + (t & 15)));
+            bool nan = false;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) nan |= __builtin_isnan(static_cast<float>(x0[e]));
+            return nan;
+        },
+        [&](int tok, int c, float) { return plane_value(xs, tok, c, n_blk); });
 }
 
 // The segment holding a row: selected field by field (an index into the
@@ -739,16 +784,33 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
                 for (int w = 0; w < kWaves; ++w) s2 += s_ss[w][(4 * g + (c & 3) + kTok * u) & 15];
             rms = 1.0f / sqrtf(s2 / static_cast<float>(p.cols) + p.eps);
         }
-        if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
-            // (normalised value by value: 1 / rms may be zero for a finite row)
+        const bool redo = ok && !(fabsf(sum) < __builtin_huge_valf());
+        if (__builtin_expect(__any(redo), 0)) {
             const unsigned char* const wr = rs.w + static_cast<long long>(rs.row) * p.row_bytes;
-            const float* const xr = p.x + t * p.x_stride;
-            sum = plain_sum<kType>(wr, 0, p.cols, [&](int col) {
-                return kSrc == kXPlanes ? plane_value(p.xs, t, col, n_blk) : kNorm ? xr[col] * rms * s_norm[col] : xr[col];
-            });
-        } else if constexpr (kNorm) {
-            sum *= rms;
+            if constexpr (kSrc == kXPlanes) {
+                sum = taken_again<kType>(sum, redo, wr, t, 0, p.cols, p.xs, n_blk);
+            } else {
+                // normalised value by value: 1 / rms may be zero for a finite
+                // row, and makes an infinity NaN
+                const int tok = min(t, p.n - 1);
+                sum = taken_again<kType>(
+                    sum, redo, wr, tok, rms, 0, p.cols,
+                    [&](int c8) {
+                        float v[8];
+                        load8(p.x + tok * p.x_stride + 8 * c8, v);
+                        bool bad = false;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            bad |= kNorm ? !(fabsf(v[e]) < __builtin_huge_valf()) : __builtin_isnan(v[e]);
+                        return bad;
+                    },
+                    [&](int of, int c, float scale) {
+                        const float v = p.x[of * p.x_stride + c];
+                        return kNorm ? v * scale * s_norm[c] : v;
+                    });
+            }
         }
+        if constexpr (kNorm) sum = redo ? sum : sum * rms;
         if (ok && rs.out) {
             float* const o = rs.out + rs.row + t * rs.stride;
             *o = p.add ? *o + sum : sum;
@@ -895,10 +957,13 @@ __global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const Pro
                 for (int w = 1; w < kWaves; ++w) sum += s_red[buf][w][c][lane];
                 const int t = 16 * tile + 4 * g + (c & 3);
                 const bool ok = row_ok[i] && t < p.n;
-                if (ok && !(fabsf(sum) < __builtin_huge_valf())) {
-                    const TileRow rs = tile_row(p, sub0 + (c >> 2), j);
-                    sum = plain_sum<kType>(rs.w + static_cast<long long>(rs.row) * p.row_bytes, 32 * kb_lo, 32 * kb_hi,
-                                           [&](int col) { return plane_value(p.xs, t, col, n_blk); });
+                const bool redo = ok && !(fabsf(sum) < __builtin_huge_valf());
+                if (__builtin_expect(__any(redo), 0)) {
+                    int j_here = j;
+                    asm volatile("" : "+v"(j_here));
+                    const TileRow rs = tile_row(p, sub0 + (c >> 2), j_here);
+                    sum = taken_again<kType>(sum, redo, rs.w + static_cast<long long>(rs.row) * p.row_bytes, t,
+                                             32 * kb_lo, 32 * kb_hi, p.xs, n_blk);
                 }
                 if (ok && out[i]) {
                     float* const o = out[i] + t * stride[i];
@@ -1124,17 +1189,18 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
         store(std::false_type{});
         return;
     }
-    unsigned redo = store(std::true_type{});
+    const unsigned redo = store(std::true_type{});
 #pragma unroll 1
-    while (redo) {
-        const int i = __builtin_ctz(redo), row = row0 + (i >> 4) * 16 + j;
-        const int t = 16 * (s0 + (i >> 2 & 3)) + 4 * g + (i & 3);
-        redo &= redo - 1;
+    for (int i = 0; i < 16 * kRW; ++i) {
+        const bool mine = redo >> i & 1;
+        if (!__any(mine)) continue;
+        const int row = min(row0 + 16 * (i >> 4) + j, p.total_rows - 1), t = 16 * (s0 + (i >> 2 & 3)) + 4 * g + (i & 3);
+        const RowSeg rs = row_seg(p, row);
+        const float sum = taken_again<kType>(0.f, mine, rs.w + static_cast<long long>(rs.row) * p.row_bytes, t, 32 * kb_lo,
+                                             32 * kb_hi, p.xs, n_blk);
+        if (!mine) continue;
         long long stride;
         float* const o = target(row, stride) + t * stride;
-        const RowSeg rs = row_seg(p, row);
-        const float sum = plain_sum<kType>(rs.w + static_cast<long long>(rs.row) * p.row_bytes, 32 * kb_lo, 32 * kb_hi,
-                                           [&](int col) { return plane_value(p.xs, t, col, n_blk); });
         *o = add ? *o + sum : sum;
     }
 }
