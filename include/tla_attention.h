@@ -441,15 +441,18 @@ enum tla_option {
                                  length: 1, 2 or 4 (the other plan always takes 4);
                                  results do not depend on it */
     TLA_OPT_STREAM_TILES = 3, /* batched products that keep their weights in registers:
-                                 token tiles of 16 per workgroup, at most, 1 to 4;
-                                 results do not depend on it */
+                                 token tiles of 16 per workgroup, at most, 1 to 4 (0:
+                                 per shape); results do not depend on it */
     TLA_OPT_SPLIT_ROWS = 4,   /* batched products: 16-row subtiles per workgroup
                                  or wave, 1, 2 or 4 (0: per shape; at most what the
-                                 format allows); results do not depend on it */
-    TLA_OPT_SPLIT_K = 5       /* the same products: ranges K is cut into, 1 to 64
-                                 (0: per shape; at least one per 2048 columns, at
-                                 most one per 64; products that split x themselves
-                                 take one); results change by fp32 rounding only */
+                                 format allows, and one where four blocks of up to 4
+                                 vectors share an operand); results do not depend on
+                                 it */
+    TLA_OPT_SPLIT_K = 5       /* the same products: ranges K is cut into, 1 to 64 (0:
+                                 per shape; at most one per 64 columns; products that
+                                 keep their weights in registers cut at least one per
+                                 2048 columns, those that split x themselves take
+                                 one); results change by fp32 rounding only */
 };
 enum tla_decode_plan { TLA_PLAN_AUTO = 0, TLA_PLAN_ALIGNED = 1, TLA_PLAN_BALANCED = 2 };
 int tla_set_option(tla_engine* e, int option, long long value);

@@ -71,6 +71,41 @@ def test_product_infinities_many_tokens(W, engines, t, name, n, rows, cols):
     infinities(W, engines(1, 64), t, name, n, rows, cols)
 
 
+# direct: four blocks to an x operand (one subtile by shape) and two (three
+# subtiles by shape); resident; tiled in the K ranges of its shape
+OPTION_SHAPES = [(2048, 2048, 3), (300, 3136, 4), (11264, 2048, 3), (9000, 1344, 4), (4112, 1024, 33), (2064, 4352, 300),
+                 (8208, 256, 250), (11264, 2048, 100)]
+
+
+@pytest.mark.parametrize("t,name", TYPES)
+@pytest.mark.parametrize("rows,cols,n", OPTION_SHAPES)
+def test_tiling_options_keep_the_bits(tla, W, engines, t, name, rows, cols, n):
+    """Row subtiles and token tiles per workgroup change no bit of a product,
+    with K cut as the shape has it."""
+    if t == Q.Q6_K and cols % 256:
+        pytest.skip("Q6_K rows are whole 256-weight super-blocks")
+    eng = engines(1, 64)
+    raw = W.make_weights(t, rows, cols, salt=rows + cols)
+    x = np.random.default_rng(n + rows).standard_normal((n, cols)).astype(np.float32)
+    with device_arrays() as track:
+        w, xd, out = track(eng.array(raw)), track(eng.array(x)), track(eng.array((n, rows)))
+
+        def product():
+            out.upload(np.full((n, rows), np.nan, np.float32))
+            eng.matmul_batch(out.ptr, w.ptr, xd.ptr, rows, cols, n, t)
+            return out.download()
+
+        base = product()
+        for opt, values in ((tla.OPT_SPLIT_ROWS, (1, 2, 4)), (tla.OPT_STREAM_TILES, (1, 3))):
+            try:
+                for v in values:
+                    eng.set_option(opt, v)
+                    assert np.array_equal(product().view(np.uint32), base.view(np.uint32)), (opt, v)
+            finally:
+                eng.set_option(opt, 0)
+    rows_close(base, raw, x, t, rows, cols, 1e-5, f"{name} {rows}x{cols} x {n}")
+
+
 @pytest.mark.parametrize("n,rows,cols", [(12, 2048, 5632), (512, 11264, 2048)])
 def test_nan_token_costs_little(W, engines, n, rows, cols):
     """A token with a NaN does not hold up the batch it is in: the product stays

@@ -337,7 +337,7 @@ def test_split_product_tilings(tla, O, W, engines, t, name, rows, cols, n_tok):
         xd = track(eng.array(x))
         out = track(eng.array((n_tok, rows)))
         try:
-            # row tilings with K fixed (the per-shape K split follows the tiling)
+            # row tilings with K in three ranges
             eng.set_option(tla.OPT_SPLIT_K, 3)
             for v in (1, 2, 4):
                 eng.set_option(tla.OPT_SPLIT_ROWS, v)

@@ -38,6 +38,7 @@ struct ProductParams {
     int n_tiles;               // token tiles of 16 (tiled: a multiple of 4)
     int rows_per_group;        // 16-row subtiles per workgroup (tiled: per wave)
     int row_groups;
+    int x_share;               // direct: consecutive blocks that share an x operand, 1, 2 or 4
     int shares;                // resident: workgroups per row group and K range, each a share of the tiles
     int k_splits;              // K cut into this many ranges of blk_per_split 32-column
     int blk_per_split;         // blocks (even); each range's sums go to part, and a
@@ -48,6 +49,7 @@ struct ProductParams {
 // Fills the plan from the shape (n, total_rows, cols, pair) for n_cu compute
 // units; the options (0: per shape) are the row subtiles per workgroup, the
 // token tiles per resident workgroup (at most) and the K ranges (at least).
+// The first two leave every sum's order as it is.
 void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p);
 hipError_t launch_product(int type, const ProductParams& p, hipStream_t s);
 

@@ -44,8 +44,9 @@
 //   tiled     past 192 tokens for the shapes whose decoded weights are too
 //             many for the registers: a 64 kRW row x 64 token tile per
 //             workgroup, x through LDS.
-// Every output is a sum in a fixed order: the same bits on every run and for
-// any grid.
+// Every output is a sum in a fixed order, which the shape, the CU count and
+// TLA_OPT_SPLIT_K choose: the same bits on every run and for any tiling of the rows
+// and tokens.
 #include <algorithm>
 #include <type_traits>
 
@@ -1262,18 +1263,13 @@ hipError_t launch_direct_share(const ProductParams& p, hipStream_t s)
     }
 }
 
-// Up to 8 tokens two blocks share an x operand, up to 4 tokens four: with one
-// row subtile (the accumulators of four for three subtiles leave no registers
-// for loads: F32, 11264 x 2048, 3 tokens 28 against 18 us; Q4_0, 32000 rows, 26
-// against 22) and more than one group of them per wave (900 x 1024, F16 4.5
-// against 4.3 us).
 template <int kType, int kR>
 hipError_t launch_direct(const ProductParams& p, hipStream_t s)
 {
     if constexpr (kR <= direct_rows(kType)) {
         if constexpr (kR == 1)
-            if (p.n <= 4 && p.cols / 32 > 4 * kWaves) return launch_direct_share<kType, kR, 4>(p, s);
-        return p.n <= 8 ? launch_direct_share<kType, kR, 2>(p, s) : launch_direct_share<kType, kR, 1>(p, s);
+            if (p.x_share == 4) return launch_direct_share<kType, kR, 4>(p, s);
+        return p.x_share == 2 ? launch_direct_share<kType, kR, 2>(p, s) : launch_direct_share<kType, kR, 1>(p, s);
     } else {
         return hipErrorInvalidValue;
     }
@@ -1330,6 +1326,7 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
     p->n_tiles = tiles;
     p->k_splits = 1;
     p->blk_per_split = n_blk;
+    p->x_share = 1;
     p->shares = 1;
     // Up to 16 tokens, or where the row subtiles and token tiles fit the CUs
     // in one round: no launch for the planes.  As many rows per workgroup as
@@ -1341,7 +1338,15 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         int r = 1;
         while (r < direct_rows(type) && static_cast<long long>((sub + r - 1) / r) * tiles > n_cu) ++r;
         if (static_cast<long long>((sub + r - 1) / r) * tiles > n_cu) r = 2;
-        if (opt_rows > 0) r = std::min(opt_rows, direct_rows(type));
+        // Up to 8 tokens two blocks share an x operand, up to 4 tokens four:
+        // with one row subtile (the accumulators of four for three subtiles
+        // leave no registers for loads: F32, 11264 x 2048, 3 tokens 28 against
+        // 18 us; Q4_0, 32000 rows, 26 against 22) and more than one group of
+        // them per wave (900 x 1024, F16 4.5 against 4.3 us).  The choice is the
+        // shape's: it sets the order of the sums, so the row option, which
+        // does not, leaves four blocks their one subtile.
+        p->x_share = p->n <= 4 && r == 1 && n_blk > 4 * kWaves ? 4 : p->n <= 8 ? 2 : 1;
+        if (opt_rows > 0 && p->x_share < 4) r = std::min(opt_rows, direct_rows(type));
         p->rows_per_group = r;
         p->row_groups = (sub + r - 1) / r;
         return;
@@ -1362,13 +1367,13 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         // ranges of at least 8 blocks.
         const auto groups = [&](int r) { return (p->total_rows + 64LL * r - 1) / (64LL * r) * (p->n_tiles / kTW); };
         int r = 2 * groups(2) >= n_cu ? 2 : 1;
-        if (opt_rows > 0) r = std::min(opt_rows, 2);
-        p->rows_per_group = r;
-        p->row_groups = (p->total_rows + 64 * r - 1) / (64 * r);
         const long long target = 5LL * n_cu / 2;
         splits = static_cast<int>(std::min<long long>((target + groups(r) - 1) / groups(r), n_blk / 8));
         if (opt_k > 0) splits = std::min(opt_k, n_blk / 2);
         splits = std::max(1, splits);
+        if (opt_rows > 0) r = std::min(opt_rows, 2);  // (the ranges stay the shape's)
+        p->rows_per_group = r;
+        p->row_groups = (p->total_rows + 64 * r - 1) / (64 * r);
     } else {
         p->kind = kProductResident;
         // The rows per workgroup and the shares of the token tiles with the
@@ -1462,7 +1467,8 @@ hipError_t launch_product(int type, const ProductParams& p, hipStream_t s)
     bool fits = false;
     switch (p.kind) {
     case kProductDirect:
-        fits = r <= direct_rows(type) && p.row_groups == (sub + r - 1) / r && p.n_tiles == tiles && p.k_splits == 1;
+        fits = (p.x_share == 1 || (p.x_share == 2 && p.n <= 8) || (p.x_share == 4 && p.n <= 4 && r == 1)) &&
+               r <= direct_rows(type) && p.row_groups == (sub + r - 1) / r && p.n_tiles == tiles && p.k_splits == 1;
         break;
     case kProductResident:
         fits = r <= resident_rows(type) && p.row_groups == (sub + r - 1) / r && p.n_tiles == tiles &&
