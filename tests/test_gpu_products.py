@@ -81,7 +81,8 @@ OPTION_SHAPES = [(2048, 2048, 3), (300, 3136, 4), (11264, 2048, 3), (9000, 1344,
 @pytest.mark.parametrize("rows,cols,n", OPTION_SHAPES)
 def test_tiling_options_keep_the_bits(tla, W, engines, t, name, rows, cols, n):
     """Row subtiles and token tiles per workgroup change no bit of a product,
-    with K cut as the shape has it."""
+    with K cut as the shape has it; one token tile per workgroup takes more than
+    eight workgroups per row group where there are more tiles."""
     if t == Q.Q6_K and cols % 256:
         pytest.skip("Q6_K rows are whole 256-weight super-blocks")
     eng = engines(1, 64)

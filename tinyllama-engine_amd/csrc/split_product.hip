@@ -1385,9 +1385,9 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         for (int r = 1; r <= most; ++r) {
             if (opt_rows > 0 && r != std::min(opt_rows, most)) continue;
             const long long groups = static_cast<long long>((sub + r - 1) / r) * splits;
-            for (int shares = 1; shares <= std::min(tiles, 8); ++shares) {
+            for (int shares = 1; shares <= (opt_tiles > 0 ? tiles : std::min(tiles, 8)); ++shares) {
                 const int each = (tiles + shares - 1) / shares;
-                if (opt_tiles > 0 && shares < std::min(tiles, 8) && each > opt_tiles) continue;
+                if (opt_tiles > 0 && each > opt_tiles) continue;
                 const double rounds = static_cast<double>((groups * shares + n_cu - 1) / n_cu);
                 const double cost = rounds * (3.0 + 1.5 * r + each * (1.6 + 0.17 * r));
                 if (best == 0 || cost < best) {
