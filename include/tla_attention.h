@@ -199,7 +199,9 @@ int tla_decode_noalloc(tla_engine* e, int n_seq, const int* pos_host, int layer0
  * Engine memory it keeps for later calls: the keys and values of positions
  * 0 .. pos0+n_tok-1 as bf16 planes, n_step_layers x n_head_kv x
  * ceil((pos0 + n_tok) / 32) x 24 KiB, grown (after a stream synchronize) when
- * a call needs more. */
+ * a call needs more -- not for short prompts, or few tokens after a long context,
+ * which run as one launch -- and 51 MiB for launches whose query tiles are
+ * shared by several workgroups, allocated by the first of them. */
 int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layers, int flags,
                 float* out_dev, const float* q_dev, const float* k_dev, const float* v_dev,
                 float* key_cache_dev, float* value_cache_dev);

@@ -7,6 +7,8 @@ kernel with 1, 2, 3 and 5 workgroups to a query tile, head groups of 1, 2 and
 Tolerance: as test_gpu_prefill.py (1e-4 on outputs; cache bit-exact).  The
 states of a query tile are merged in a fixed order, so a second call gives
 the same bits."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -69,3 +71,36 @@ def test_prefill_rows_already_in_the_cache(W, engines, pos0, n_tok):
         eng.prefill(pos0, n_tok, 0, 1, q.ptr, q.ptr, dkc.ptr + off, dvc.ptr + off, dkc.ptr, dvc.ptr)
         assert max_err(q.download(), out) <= PREFILL_TOL
         assert np.array_equal(bits(dkc.download()), bits(kc)) and np.array_equal(bits(dvc.download()), bits(vc))
+
+
+def free_bytes(tla):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert tla.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("layers,pos0,n_tok,shared", [(1, 0, 20, False), (22, 0, 200, False), (1, 300, 1, True)])
+def test_prefill_allocates_what_it_uses(tla, W, layers, pos0, n_tok, shared):
+    """The workspace of shared query tiles (51 MiB) comes with the first launch
+    that shares one, not with a launch that does not; the planes with a launch
+    that reads them."""
+    n_ctx = pos0 + n_tok
+    case = W.make_prefill(n_layers=layers, n_tok=n_tok, pos0=pos0, salt=1)
+    eng = tla.Engine(tla.Config(layers, 2048, 32, 4, n_ctx, 10000.0))
+    try:
+        with device_arrays() as track:
+            q, k, v = (track(eng.array(a)) for a in (case.q, case.k, case.v))
+            out = track(eng.array(case.q.shape))
+            kc, vc = eng.kv_cache(1)
+            track(kc), track(vc)
+            eng.synchronize()
+            before = free_bytes(tla)
+            for _ in range(2):
+                eng.prefill(pos0, n_tok, 0, layers, out.ptr, q.ptr, k.ptr, v.ptr, kc.ptr, vc.ptr)
+            eng.synchronize()
+            used = before - free_bytes(tla)
+    finally:
+        eng.close()
+    planes = layers * 4 * ((n_ctx + 31) // 32) * 24576 if layers > 1 else 0
+    log(f"    {used >> 20} MiB")
+    assert used - planes < 8 << 20 if not shared else 51 << 20 <= used < 60 << 20

@@ -276,8 +276,7 @@ int ensure_prefill_part(tla_engine* e)
     void* buf = nullptr;
     TLA_HIP(hipMalloc(&buf, states + counters));
     int* const cnt = reinterpret_cast<int*>(static_cast<char*>(buf) + states);
-    hipError_t rc = launch_zero(cnt, counters, e->stream);
-    if (rc == hipSuccess) rc = hipStreamSynchronize(e->stream);
+    const hipError_t rc = launch_zero(cnt, counters, e->stream);  // ahead of the launch that counts
     if (rc != hipSuccess) {
         (void)hipFree(buf);
         TLA_HIP(rc);
@@ -1227,7 +1226,6 @@ int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layer
     p.gqa = e->gqa;
     p.rotate = (flags & TLA_ROTATE) ? 1 : 0;
     p.scale_log2 = scale_log2(e->head_dim);
-    if (int rc = ensure_prefill_part(e)) return rc;
     // One launch reads inputs and cache while it writes cache and output: a
     // caller whose buffers overlap (k and v rows already in their place in the
     // cache, say) keeps the two launches, where the rows are read before they
@@ -1242,7 +1240,10 @@ int tla_prefill(tla_engine* e, int pos0, int n_tok, int layer0, int n_step_layer
     }
     for (const float* cache : caches)
         apart &= !overlap(q_dev, n_out, cache, n_cache) && !overlap(out_dev, n_out, cache, n_cache);
-    if (apart && prefill_is_short(n_step_layers, c.n_head_kv, e->gqa, pos0, n_tok))
+    const bool one_launch = apart && prefill_is_short(n_step_layers, c.n_head_kv, e->gqa, pos0, n_tok);
+    if (prefill_shares(one_launch, n_step_layers, c.n_head_kv, e->gqa, pos0, n_tok))
+        if (int rc = ensure_prefill_part(e)) return rc;
+    if (one_launch)
         return launch(e, TLA_KERNEL_PREFILL, "prefill",
                       [&] { return launch_prefill_short(p, e->pf_part, e->pf_counters, e->stream); });
     p.n_ptiles = (pos0 + n_tok + 31) / 32;

@@ -955,9 +955,9 @@ bool prefill_is_short(int n_lb, int n_head_kv, int gqa, int pos0, int n_tok)
 
 hipError_t launch_prefill_short(const PrefillParams& p, float* part, int* counters, hipStream_t s)
 {
-    if (!prefill_is_short(p.n_lb, p.n_head_kv, p.gqa, p.pos0, p.n_tok) || !part || !counters)
-        return hipErrorInvalidValue;
+    if (!prefill_is_short(p.n_lb, p.n_head_kv, p.gqa, p.pos0, p.n_tok)) return hipErrorInvalidValue;
     const ShortShape h = short_shape(p.n_lb, p.n_head_kv, p.gqa, p.pos0, p.n_tok);
+    if (h.n_ch > 1 && (!part || !counters)) return hipErrorInvalidValue;
     const ShortGrid g{h.n_hg, h.heads, part, counters};
     const dim3 grid(h.n_qt, h.n_ch, (unsigned)h.z);
     if (h.stage == 1)
@@ -995,15 +995,27 @@ int attention_chunks(long long units, int n_kt)
     return n > 1 && units <= kPrefillCounters && units * n * kWavesP <= kPrefillStates ? (int)n : 1;
 }
 
+int planes_chunks(int n_lb, int n_head_kv, int gqa, int pos0, int n_tok)
+{
+    const long long units =
+        (long long)n_lb * n_head_kv * ((gqa + kWavesP - 1) / kWavesP) * ((n_tok + kQTile - 1) / kQTile);
+    return attention_chunks(units, (pos0 + n_tok + kKTile - 1) / kKTile);
+}
+
 }  // namespace
+
+bool prefill_shares(bool short_launch, int n_lb, int n_head_kv, int gqa, int pos0, int n_tok)
+{
+    return (short_launch ? short_shape(n_lb, n_head_kv, gqa, pos0, n_tok).n_ch
+                         : planes_chunks(n_lb, n_head_kv, gqa, pos0, n_tok)) > 1;
+}
 
 hipError_t launch_prefill_attention(const PrefillParams& p, float* part, int* counters, hipStream_t s)
 {
-    if (!p.kvp || p.n_ptiles != (p.pos0 + p.n_tok + kKTile - 1) / kKTile || !part || !counters)
+    const int n_ch = planes_chunks(p.n_lb, p.n_head_kv, p.gqa, p.pos0, p.n_tok);
+    if (!p.kvp || p.n_ptiles != (p.pos0 + p.n_tok + kKTile - 1) / kKTile || (n_ch > 1 && (!part || !counters)))
         return hipErrorInvalidValue;
-    const long long pairs = (long long)p.n_lb * p.n_head_kv;
-    const long long units = pairs * ((p.gqa + kWavesP - 1) / kWavesP) * ((p.n_tok + kQTile - 1) / kQTile);
-    return launch_attention(p, attention_chunks(units, p.n_ptiles), part, counters, s);
+    return launch_attention(p, n_ch, part, counters, s);
 }
 
 }  // namespace tla
