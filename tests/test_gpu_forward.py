@@ -629,6 +629,39 @@ def test_prefill_forward_split_prompt(tla, O, W, engines, name):
         assert np.abs(kd[0, :, :n] - ok[:, :n]).max() <= 1e-4 * np.abs(ok[:, :n]).max()
 
 
+# n_ff 2304: W_down in K ranges whose sums the next layer's norm adds to x (40
+# tokens: resident products; 170: tiled, F16 gate and up too, unpaired); n_embd
+# 2304: W_o in ranges, added by the FFN's norm, whose rows take two passes of a
+# workgroup
+@pytest.mark.parametrize("wtype,n,shape", [
+    (Q.Q8_0, 40, (512, 8, 2, 2304)), (Q.Q4_0, 170, (512, 8, 2, 2304)), (Q.F16, 170, (512, 8, 2, 2304)),
+    (Q.Q4_0, 90, (2304, 36, 12, 512)), (Q.F16, 90, (2304, 36, 12, 512))])
+def test_prefill_forward_wide_layers(tla, O, W, engines, wtype, n, shape):
+    """Two layers with rows of more than 2048 columns: logits of the last token
+    and every K and V row against the oracle's token loop."""
+    embd, n_head, n_head_kv, ff = shape
+    spec = W.ModelSpec(2, embd, n_head, n_head_kv, ff, 512, 192)
+    t = W.make_model(spec, wtype, salt=91)
+    eng = spec_engine(engines, spec)
+    toks = np.random.default_rng(n).integers(0, spec.n_vocab, n).tolist()
+    om = O.Model(spec, t)
+    want = om.tokens(toks)[-1]
+    dm = tla.DeviceModel(eng, t, spec.n_ff, spec.n_vocab, spec.rms_norm_eps)
+    try:
+        with device_arrays() as track:
+            kc, vc = eng.kv_cache(1)
+            track(kc), track(vc)
+            lg = track(eng.array((spec.n_vocab,)))
+            eng.prefill_forward(dm, kc.ptr, vc.ptr, toks, 0, lg.ptr)
+            got, caches = lg.download(), (kc.download(), vc.download())
+    finally:
+        dm.free()
+    check_logits(got[None], want[None], f"n_embd {embd}, n_ff {ff}, {n} tokens vs oracle")
+    for dev, host in zip(caches, (om.kc, om.vc)):
+        ref = host.reshape(spec.n_layers, spec.n_ctx, spec.kv_dim)
+        assert np.abs(dev[0, :, :n] - ref[:, :n]).max() <= 1e-4 * np.abs(ref[:, :n]).max()
+
+
 def test_prefill_forward_after_queued_weight_writes(tla, O, W, engines):
     """Weights written on the engine's stream and not yet synchronized when a
     prompt starts: every product of the prompt must see them.  Layers 0 and

@@ -183,8 +183,22 @@ def test_layer_halves(O, W, engines, t, name, n):
     """tla_attn_qkv (with its rmsnorm), tla_attn_out and tla_ffn_block over n
     sequences: the norm and SwiGLU fused where the shape allows, gate and up
     left in hb as they were before."""
-    eng = engines(1, 64, 8, 2)
-    embd, kv, ff = 512, 128, 768
+    layer_halves(O, W, engines(1, 64, 8, 2), t, name, n, 768)
+
+
+# n_ff 2304: W_down in several K ranges from the planes of silu(gate) * up (n 40),
+# which a launch of its own writes where gate and up take the tiled product (F16 and F32
+# from 81); n_embd 2304: norms of more columns than one pass of a workgroup
+@pytest.mark.parametrize("t,name,n,n_head,n_head_kv,n_ff", [
+    (Q.Q8_0, "q8_0", 40, 8, 2, 2304), (Q.Q6_K, "q6_k", 40, 8, 2, 2304), (Q.F16, "f16", 100, 8, 2, 2304),
+    (Q.F32, "f32", 100, 8, 2, 2304), (Q.Q4_0, "q4_0", 170, 8, 2, 2304), (Q.Q8_0, "q8_0", 40, 36, 12, 768),
+    (Q.F16, "f16", 12, 36, 12, 768)])
+def test_layer_halves_wide(O, W, engines, t, name, n, n_head, n_head_kv, n_ff):
+    layer_halves(O, W, engines(1, 64, n_head, n_head_kv), t, name, n, n_ff)
+
+
+def layer_halves(O, W, eng, t, name, n, ff):
+    embd, kv = eng.cfg.n_embd, 64 * eng.cfg.n_head_kv
     wq, wk, wv = (W.make_weights(t, r, embd, salt=i) for i, r in ((1, embd), (2, kv), (3, kv)))
     wo = W.make_weights(t, embd, embd, salt=4)
     wg, wu = W.make_weights(t, ff, embd, salt=5), W.make_weights(t, ff, embd, salt=6)
