@@ -629,13 +629,13 @@ def test_prefill_forward_split_prompt(tla, O, W, engines, name):
         assert np.abs(kd[0, :, :n] - ok[:, :n]).max() <= 1e-4 * np.abs(ok[:, :n]).max()
 
 
-# n_ff 2304: W_down in K ranges whose sums the next layer's norm adds to x (40
-# tokens: resident products; 170: tiled, F16 gate and up too, unpaired); n_embd
-# 2304: W_o in ranges, added by the FFN's norm, whose rows take two passes of a
-# workgroup
+# n_ff 2304: W_down in two K ranges, whose sums the next layer's norm adds to x;
+# n_ff 4352: it and the unpaired gate and up are tiled products; n_embd 2304: W_o
+# in ranges (Q4_0 resident, F32 tiled), added by the FFN's norm, whose rows take
+# two passes of a workgroup
 @pytest.mark.parametrize("wtype,n,shape", [
-    (Q.Q8_0, 40, (512, 8, 2, 2304)), (Q.Q4_0, 170, (512, 8, 2, 2304)), (Q.F16, 170, (512, 8, 2, 2304)),
-    (Q.Q4_0, 90, (2304, 36, 12, 512)), (Q.F16, 90, (2304, 36, 12, 512))])
+    (Q.Q8_0, 170, (512, 8, 2, 2304)), (Q.F16, 170, (512, 8, 2, 2304)), (Q.F32, 170, (1024, 16, 4, 4352)),
+    (Q.Q4_0, 90, (2304, 36, 12, 512)), (Q.F32, 90, (2304, 36, 12, 512))])
 def test_prefill_forward_wide_layers(tla, O, W, engines, wtype, n, shape):
     """Two layers with rows of more than 2048 columns: logits of the last token
     and every K and V row against the oracle's token loop."""

@@ -66,7 +66,7 @@ def test_product_infinities(W, engines, t, name, n, rows):
 # where the tiled product runs: F16 and F32 in one K range, every format but
 # Q6_K (which keeps the resident one) in several
 @pytest.mark.parametrize("t,name", TYPES)
-@pytest.mark.parametrize("n,rows,cols", [(130, 4128, 256), (170, 72, 2304)])
+@pytest.mark.parametrize("n,rows,cols", [(250, 8208, 256), (300, 2064, 4352)])
 def test_product_infinities_many_tokens(W, engines, t, name, n, rows, cols):
     infinities(W, engines(1, 64), t, name, n, rows, cols)
 
@@ -186,12 +186,12 @@ def test_layer_halves(O, W, engines, t, name, n):
     layer_halves(O, W, engines(1, 64, 8, 2), t, name, n, 768)
 
 
-# n_ff 2304: W_down in several K ranges from the planes of silu(gate) * up (n 40),
-# which a launch of its own writes where gate and up take the tiled product (F16 and F32
-# from 81); n_embd 2304: norms of more columns than one pass of a workgroup
+# n_ff 2304: W_down in two K ranges from the planes of silu(gate) * up; n_ff 4352:
+# gate and up take the tiled product, and a launch of its own writes the planes;
+# n_embd 2304: norms of more columns than one pass of a workgroup
 @pytest.mark.parametrize("t,name,n,n_head,n_head_kv,n_ff", [
-    (Q.Q8_0, "q8_0", 40, 8, 2, 2304), (Q.Q6_K, "q6_k", 40, 8, 2, 2304), (Q.F16, "f16", 100, 8, 2, 2304),
-    (Q.F32, "f32", 100, 8, 2, 2304), (Q.Q4_0, "q4_0", 170, 8, 2, 2304), (Q.Q8_0, "q8_0", 40, 36, 12, 768),
+    (Q.Q8_0, "q8_0", 170, 8, 2, 2304), (Q.Q6_K, "q6_k", 170, 8, 2, 2304), (Q.F16, "f16", 170, 16, 4, 4352),
+    (Q.F32, "f32", 100, 16, 4, 4352), (Q.Q4_0, "q4_0", 170, 8, 2, 2304), (Q.Q8_0, "q8_0", 40, 36, 12, 768),
     (Q.F16, "f16", 12, 36, 12, 768)])
 def test_layer_halves_wide(O, W, engines, t, name, n, n_head, n_head_kv, n_ff):
     layer_halves(O, W, engines(1, 64, n_head, n_head_kv), t, name, n, n_ff)
