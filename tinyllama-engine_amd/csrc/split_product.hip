@@ -1139,18 +1139,9 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
     __builtin_amdgcn_s_waitcnt(0);
 
     // lane (g, j) holds tokens 16 (s0 + s) + 4 g + q of row row0 + 16 r + j;
-    // with K split, the sums go to part[z][t][row] for range_sum_kernel
-    const auto target = [&](int row, long long& stride) __attribute__((always_inline)) {
-        if (p.part) {
-            stride = p.total_rows;
-            return p.part + static_cast<long long>(tz) * p.n * p.total_rows + row;
-        }
-        const RowSeg rs = row_seg(p, row);
-        stride = rs.stride;
-        return rs.out + rs.row;
-    };
-    const bool add = p.add && !p.part;
-    // Sums that are not finite are left out (bit 16 r + 4 s + q of the result).
+    // with K split, the sums go to part[z][t][row] for range_sum_kernel.  Checked:
+    // sums that are not finite are left out (bit 16 r + 4 s + q of the result).
+    float* const part = p.part ? p.part + static_cast<long long>(tz) * p.n * p.total_rows : nullptr;
     const auto store = [&](auto checked) __attribute__((always_inline)) {
         unsigned redo = 0;
         static_assert(kRW * kTW * 4 <= 32, "one bit per sum");
@@ -1158,27 +1149,33 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
         for (int r = 0; r < kRW; ++r) {
             const int row = row0 + 16 * r + j;
             if (row >= p.total_rows) continue;
-            long long stride;
-            float* const out = target(row, stride);
+            const auto rows = [&](float* out, long long stride, bool add) __attribute__((always_inline)) {
 #pragma unroll
-            for (int s = 0; s < kTW; ++s)
+                for (int s = 0; s < kTW; ++s)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int t = 16 * (s0 + s) + 4 * g + q;
-                    if (t >= p.n) continue;
-                    if (checked && !(fabsf(acc[r][s][q]) < __builtin_huge_valf())) {
-                        redo |= 1u << (16 * r + 4 * s + q);
-                        continue;
+                    for (int q = 0; q < 4; ++q) {
+                        const int t = 16 * (s0 + s) + 4 * g + q;
+                        if (t >= p.n) continue;
+                        if (checked && !(fabsf(acc[r][s][q]) < __builtin_huge_valf())) {
+                            redo |= 1u << (16 * r + 4 * s + q);
+                            continue;
+                        }
+                        float* const o = out + static_cast<long long>(t) * stride;
+                        *o = add ? *o + acc[r][s][q] : acc[r][s][q];
                     }
-                    float* const o = out + static_cast<long long>(t) * stride;
-                    *o = add ? *o + acc[r][s][q] : acc[r][s][q];
-                }
+            };
+            if (part) {
+                rows(part + row, p.total_rows, false);
+                continue;
+            }
+            const RowSeg rs = row_seg(p, row);
+            rows(rs.out + rs.row, rs.stride, p.add);
         }
         return redo;
     };
     // Zero times every sum is zero unless one is not finite: one branch for the
-    // wave (F16, 11264 x 2048, 100 tokens 42.7 -> 43.9 us, most shapes less than
-    // 1 %; a branch before each store was 1-4 %).
+    // wave (F16, 11264 x 2048, 100 tokens 42.9 -> 43.4 us; a branch before each
+    // store was 1-4 % of most shapes).
     floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < kRW; ++r)
@@ -1200,9 +1197,12 @@ __global__ __launch_bounds__(kTileThreads) void tiled_product_kernel(const Produ
         const float sum = taken_again<kType>(0.f, mine, rs.w + static_cast<long long>(rs.row) * p.row_bytes, t, 32 * kb_lo,
                                              32 * kb_hi, p.xs, n_blk);
         if (!mine) continue;
-        long long stride;
-        float* const o = target(row, stride) + t * stride;
-        *o = add ? *o + sum : sum;
+        if (part) {
+            part[static_cast<long long>(t) * p.total_rows + row] = sum;
+        } else {
+            float* const o = rs.out + rs.row + t * rs.stride;
+            *o = p.add ? *o + sum : sum;
+        }
     }
 }
 
