@@ -1,7 +1,7 @@
 """The split products of several tokens at the edges of their tiles, against
-fp64: the direct product (up to 16 tokens, or few rows), the resident one
-(more tokens; K in one or several ranges) and the tiled one (past 192
-tokens), and a layer's halves over several sequences, which run on them.
+fp64: the direct product (up to 16 tokens, or few rows), the resident and the
+tiled one (more tokens, whichever is estimated faster; K in one or several
+ranges), and a layer's halves over several sequences, which run on them.
 
 Tolerance: a row is an fp32 sum of exact products in another order than the
 reference's, |gpu - fp64| <= 1e-5 sum |w x| (test_gpu_proj.py).  A layer half
@@ -18,11 +18,12 @@ pytestmark = pytest.mark.gpu
 TYPES = [(Q.F32, "f32"), (Q.F16, "f16"), (Q.Q4_0, "q4_0"), (Q.Q8_0, "q8_0"), (Q.Q6_K, "q6_k")]
 # direct: one token tile, remainders of rows and waves, groups of four blocks
 # that the row does not fill; resident: shares of the tiles, K slices of 4 and
-# 8 blocks, two K ranges with an uneven last one; tiled: K ranges, token and
-# row remainders
+# 8 blocks, two K ranges with an uneven last one; tiled (F32 and F16 first): one
+# and several K ranges, token and row remainders
 SHAPES = [(17, 64, 3), (40, 192, 4), (4112, 1088, 2), (300, 3136, 4), (300, 3136, 5), (9000, 1344, 8),
           (50, 2368, 3), (33, 256, 6), (33, 320, 8), (4112, 256, 16), (9000, 512, 15), (4112, 1024, 17),
-          (4200, 2048, 33), (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250)]
+          (4200, 2048, 33), (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250),
+          (6160, 1024, 100), (3000, 4096, 300)]
 
 
 def rows_close(got, raw, x, t, rows, cols, tol, what):

@@ -51,6 +51,8 @@ struct ProductParams {
 // token tiles per resident workgroup (at most) and the K ranges (at least).
 // The first two leave every sum's order as it is.
 void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p);
+// Estimated microseconds of a resident or tiled plan, without the planes' launch.
+double product_us(int type, int n_cu, const ProductParams& p);
 hipError_t launch_product(int type, const ProductParams& p, hipStream_t s);
 
 hipError_t load_product_code();  // as tla_internal.h's

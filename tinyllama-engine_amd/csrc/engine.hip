@@ -820,13 +820,21 @@ int norm_product(tla_engine* e, int type, const GemvSegment* segs, int n_seg, in
 }
 
 // Whether the gate and up product of this shape runs paired (its epilogue
-// writes the planes of silu(gate) * up): where the unpaired one would not
-// take the tiled kernel, and rows are whole blocks.
+// writes the planes of silu(gate) * up, where rows are whole blocks): unless the
+// tiled product, which does not pair, is faster by more than the launch that
+// then writes the planes, less what the epilogue costs (F16, 5632 columns, a layer
+// step paired / not: 64 tokens 102.5 / 99.7 us, 96 120.4 / 129, 120 137 / 132.5).
+// By the shape, not the options.
 bool paired_product(tla_engine* e, int type, int n_ff, int cols, int n)
 {
     const GemvSegment segs[2] = {{nullptr, nullptr, n_ff, 0}, {nullptr, nullptr, n_ff, 0}};
-    return n_ff % 64 == 0 && product_params(e, type, segs, 2, cols, n, 0).kind != kProductTiled &&
-           product_params(e, type, segs, 2, cols, n, 0, true).k_splits == 1;
+    if (n_ff % 64 != 0 || product_params(e, type, segs, 2, cols, n, 0, true).k_splits != 1) return false;
+    ProductParams apart = product_params(e, type, segs, 2, cols, n, 0), pair = apart;
+    if (apart.kind != kProductTiled) return true;
+    pair.pair = 1;
+    plan_product(type, e->n_cu, 0, 0, 0, &apart);
+    plan_product(type, e->n_cu, 0, 0, 0, &pair);
+    return product_us(type, e->n_cu, pair) <= product_us(type, e->n_cu, apart) + 2 + 3e-6 * n * n_ff;
 }
 
 // x[t] += W_down . (silu(gate_t) * up_t) for n token rows, gate and up from

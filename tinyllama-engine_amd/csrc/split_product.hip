@@ -41,9 +41,9 @@
 //             x split (and normalised) by the workgroup itself;
 //   resident  more tokens: a workgroup keeps its rows' decoded weights in
 //             registers and streams the x planes of all token tiles past them;
-//   tiled     past 192 tokens for the shapes whose decoded weights are too
-//             many for the registers: a 64 kRW row x 64 token tile per
-//             workgroup, x through LDS.
+//   tiled     where its estimated time is less (many tokens; weights of several
+//             pieces, of which the registers hold few rows; several K ranges): a
+//             64 kRW row x 64 token tile per workgroup, x through LDS.
 // Every output is a sum in a fixed order, which the shape, the CU count and
 // TLA_OPT_SPLIT_K choose: the same bits on every run and for any tiling of the rows
 // and tokens.
@@ -270,7 +270,7 @@ struct Fmt {
 // compiler cannot merge), which the tiled kernel's wait for its LDS copies
 // counts.
 template <int kType>
-constexpr int kRowLoads = kType == kF32 ? 2 : kType == kQ6_K ? 4 : 1;
+constexpr int kRowLoads = kType == kF32 ? 2 : 1;
 
 template <int kType>
 __device__ __forceinline__ void load_w(WRaw<kType>& w, const unsigned char* wrow, int kb, int g)
@@ -987,11 +987,7 @@ __global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const Pro
 // wave w owns rows 16 kRW w .. + 16 kRW - 1 for all 64 tokens.  The x blocks
 // pass through a ring of three LDS stages (12 KiB each) filled by direct
 // loads two blocks ahead; each wave loads its rows' weights three blocks
-// ahead.  Bound by its barrier per block and LDS reads; kept where the
-// resident product holds too few rows or needs several K ranges (512 tokens,
-// us, tiled / resident: F16 11264 x 2048 105 / 123, F32 155 / 191, Q8_0
-// 2048 x 5632 61 / 69; 100 tokens F16 11264 x 2048 42 / 45, F32 2048 x 5632
-// 35 / 46, F32 2560 x 2048 25 / 23).  Carrying the sums
+// ahead.  Bound by its barrier per block and LDS reads.  Carrying the sums
 // of types without a scale through the matrix cores was 3-6 % faster and put a
 // layer of F16 over 100 sequences 3.6e-7 off fp64 against 1.4e-7.
 template <int kType, int kRW>
@@ -1293,10 +1289,14 @@ hipError_t launch_resident(const ProductParams& p, hipStream_t s)
 template <int kType, int kR>
 hipError_t launch_tiled(const ProductParams& p, hipStream_t s)
 {
-    const dim3 grid(static_cast<unsigned>(p.row_groups), static_cast<unsigned>(p.n_tiles / kTW),
-                    static_cast<unsigned>(p.k_splits));
-    hipLaunchKernelGGL((tiled_product_kernel<kType, kR>), grid, dim3(kTileThreads), 0, s, p);
-    return hipGetLastError();
+    if constexpr (kType == kQ6_K) {
+        return hipErrorInvalidValue;
+    } else {
+        const dim3 grid(static_cast<unsigned>(p.row_groups), static_cast<unsigned>(p.n_tiles / kTW),
+                        static_cast<unsigned>(p.k_splits));
+        hipLaunchKernelGGL((tiled_product_kernel<kType, kR>), grid, dim3(kTileThreads), 0, s, p);
+        return hipGetLastError();
+    }
 }
 
 template <int kType>
@@ -1319,6 +1319,89 @@ hipError_t launch_typed(const ProductParams& p, hipStream_t s)
 }
 
 }  // namespace
+
+namespace {
+
+// K cut into `splits` ranges of an even number of blocks.
+void cut_k(int splits, ProductParams* p)
+{
+    const int n_blk = p->cols / 32;
+    p->blk_per_split = (n_blk / 2 + splits - 1) / splits * 2;
+    p->k_splits = (n_blk + p->blk_per_split - 1) / p->blk_per_split;
+}
+
+void plan_resident(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p)
+{
+    const int n_blk = p->cols / 32, sub = (p->total_rows + 15) / 16, tiles = p->n_tiles;
+    const int splits = std::max((n_blk + kRangeBlocks - 1) / kRangeBlocks, std::min(opt_k, n_blk / 2));
+    p->kind = kProductResident;
+    // The rows per workgroup and the shares of the token tiles with the
+    // least estimated time, in microseconds: per round of workgroups, the
+    // weights (3 + 1.5 per row subtile) and each token tile (1.6 to load
+    // its planes, 0.17 per row subtile not hidden behind that).  A round that
+    // leaves CUs idle takes as long as a full one: each of its workgroups is bound
+    // by its own CU's way to the planes.
+    double best = 0;
+    const int most = resident_rows(type);
+    for (int r = 1; r <= most; ++r) {
+        if (opt_rows > 0 && r != std::min(opt_rows, most)) continue;
+        const long long groups = static_cast<long long>((sub + r - 1) / r) * splits;
+        for (int shares = 1; shares <= (opt_tiles > 0 ? tiles : std::min(tiles, 8)); ++shares) {
+            const int each = (tiles + shares - 1) / shares;
+            if (opt_tiles > 0 && each > opt_tiles) continue;
+            const double rounds = static_cast<double>((groups * shares + n_cu - 1) / n_cu);
+            const double cost = rounds * (3.0 + 1.5 * r + each * (1.6 + 0.17 * r));
+            if (best == 0 || cost < best) {
+                best = cost;
+                p->rows_per_group = r;
+                p->row_groups = (sub + r - 1) / r;
+                p->shares = shares;
+            }
+        }
+    }
+    cut_k(splits, p);
+}
+
+void plan_tiled(int n_cu, int opt_rows, int opt_k, ProductParams* p)
+{
+    const int n_blk = p->cols / 32;
+    p->kind = kProductTiled;
+    p->n_tiles = (p->n + 16 * kTW - 1) / (16 * kTW) * kTW;
+    // Two row subtiles per wave where that gives half the CUs a
+    // workgroup; K cut until the grid holds about 2.5 workgroups per CU,
+    // ranges of at least 8 blocks.
+    const auto groups = [&](int r) { return (p->total_rows + 64LL * r - 1) / (64LL * r) * (p->n_tiles / kTW); };
+    int r = 2 * groups(2) >= n_cu ? 2 : 1;
+    const long long target = 5LL * n_cu / 2;
+    int splits = static_cast<int>(std::min<long long>((target + groups(r) - 1) / groups(r), n_blk / 8));
+    if (opt_k > 0) splits = std::min(opt_k, n_blk / 2);
+    if (opt_rows > 0) r = std::min(opt_rows, 2);  // (the ranges stay the shape's)
+    p->rows_per_group = r;
+    p->row_groups = (p->total_rows + 64 * r - 1) / (64 * r);
+    cut_k(std::max(1, splits), p);
+}
+
+}  // namespace
+
+// Resident: as in plan_resident, a tile's time by its columns and by the piece
+// products per multiply-add.  Tiled: a block of a workgroup takes 0.3 where its CU
+// has no other, else the CU's workgroups share its matrix cores and LDS.  Several
+// ranges: the launch that adds their sums, a step per range, and its bytes.
+double product_us(int type, int n_cu, const ProductParams& p)
+{
+    const int products = type == kF32 ? 6 : type == kF16 || type == kQ6_K ? 5 : 3;
+    const double sums = p.k_splits > 1 ? 3.5 + 0.3 * p.k_splits + 0.8e-6 * p.n * p.total_rows * (p.k_splits + 1.0) : 0;
+    const auto rounds = [&](long long groups) { return static_cast<double>((groups + n_cu - 1) / n_cu); };
+    const int r = p.rows_per_group;
+    if (p.kind == kProductTiled) {
+        const double block = type == kF32 ? 0.36 * r : type == kF16 ? 0.26 * r : 0.08 + 0.18 * r;
+        const double per_cu = rounds(static_cast<long long>(p.row_groups) * (p.n_tiles / kTW) * p.k_splits);
+        return sums + 5 + p.blk_per_split * std::max(0.3, per_cu * block);
+    }
+    const int each = (p.n_tiles + p.shares - 1) / p.shares;
+    const double tile = (1.6 + 0.085 * products * r) * p.blk_per_split / kRangeBlocks;
+    return sums + rounds(static_cast<long long>(p.row_groups) * p.k_splits * p.shares) * (3.0 + 1.5 * r + each * tile);
+}
 
 void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p)
 {
@@ -1351,56 +1434,26 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         p->row_groups = (sub + r - 1) / r;
         return;
     }
-    const int ranges = (n_blk + kRangeBlocks - 1) / kRangeBlocks;
-    const int tiled_past = type == kF16   ? 80
-                           : type != kF32 ? 160
-                           : ranges > 1   ? 64
-                                          : p->total_rows > 4096 ? 80 : 112;
-    const bool tiled = p->n > tiled_past && type != kQ6_K && !p->pair &&
-                       (ranges > 1 || (type == kF16 && p->total_rows > 4096) || (type == kF32 && p->total_rows > 2048));
-    int splits = std::max(ranges, std::min(opt_k, n_blk / 2));
-    if (tiled) {
-        p->kind = kProductTiled;
-        p->n_tiles = (p->n + 16 * kTW - 1) / (16 * kTW) * kTW;
-        // Two row subtiles per wave where that gives half the CUs a
-        // workgroup; K cut until the grid holds about 2.5 workgroups per CU,
-        // ranges of at least 8 blocks.
-        const auto groups = [&](int r) { return (p->total_rows + 64LL * r - 1) / (64LL * r) * (p->n_tiles / kTW); };
-        int r = 2 * groups(2) >= n_cu ? 2 : 1;
-        const long long target = 5LL * n_cu / 2;
-        splits = static_cast<int>(std::min<long long>((target + groups(r) - 1) / groups(r), n_blk / 8));
-        if (opt_k > 0) splits = std::min(opt_k, n_blk / 2);
-        splits = std::max(1, splits);
-        if (opt_rows > 0) r = std::min(opt_rows, 2);  // (the ranges stay the shape's)
-        p->rows_per_group = r;
-        p->row_groups = (p->total_rows + 64 * r - 1) / (64 * r);
-    } else {
-        p->kind = kProductResident;
-        // The rows per workgroup and the shares of the token tiles with the
-        // least estimated time, in microseconds: per round of workgroups, the
-        // weights (3 + 1.5 per row subtile) and each token tile (1.6 to load
-        // its planes, 0.17 per row subtile not hidden behind that).
-        double best = 0;
-        const int most = resident_rows(type);
-        for (int r = 1; r <= most; ++r) {
-            if (opt_rows > 0 && r != std::min(opt_rows, most)) continue;
-            const long long groups = static_cast<long long>((sub + r - 1) / r) * splits;
-            for (int shares = 1; shares <= (opt_tiles > 0 ? tiles : std::min(tiles, 8)); ++shares) {
-                const int each = (tiles + shares - 1) / shares;
-                if (opt_tiles > 0 && each > opt_tiles) continue;
-                const double rounds = static_cast<double>((groups * shares + n_cu - 1) / n_cu);
-                const double cost = rounds * (3.0 + 1.5 * r + each * (1.6 + 0.17 * r));
-                if (best == 0 || cost < best) {
-                    best = cost;
-                    p->rows_per_group = r;
-                    p->row_groups = (sub + r - 1) / r;
-                    p->shares = shares;
-                }
-            }
+    // Resident or tiled by the shape's estimates (the options change no kind).
+    // Of 971 shapes measured in both kernels (F16, F32, Q4_0, Q8_0; 512 to 32000
+    // rows, 512 to 8192 columns, 20 to 1000 tokens) this takes the slower one by
+    // more than 5 % in 32 (lines of rows and tokens fitted to 2048 columns: 224),
+    // 0.4 % on average (4 %).  Us, resident / tiled: F16 8192 x 2048, 81 tokens
+    // 25.4 / 34.9, 11264 x 2048, 128 tokens 53.1 / 45.8, 8192 x 1024, 128 18.7 /
+    // 26.4; F32 4096 x 2048, 160 31.6 / 35.8, 2048 x 5632, 65 38.3 / 33.9; Q8_0
+    // 4096 x 5632, 128 46.1 / 40.6, 2048 x 4096, 256 34.3 / 35.1.  Neither a pair's
+    // epilogue nor Q6_K's decoding is in the tiled kernel.
+    ProductParams tiled = *p;
+    plan_resident(type, n_cu, 0, 0, 0, p);
+    if (!p->pair && type != kQ6_K) {
+        plan_tiled(n_cu, 0, 0, &tiled);
+        if (product_us(type, n_cu, tiled) < product_us(type, n_cu, *p)) {
+            *p = tiled;
+            if (opt_rows > 0 || opt_k > 0) plan_tiled(n_cu, opt_rows, opt_k, p);
+            return;
         }
     }
-    p->blk_per_split = (n_blk / 2 + splits - 1) / splits * 2;
-    p->k_splits = (n_blk + p->blk_per_split - 1) / p->blk_per_split;
+    if (opt_rows > 0 || opt_tiles > 0 || opt_k > 0) plan_resident(type, n_cu, opt_rows, opt_tiles, opt_k, p);
 }
 
 size_t product_planes_bytes(int n, int cols)
