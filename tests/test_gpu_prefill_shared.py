@@ -1,7 +1,7 @@
 """Prefill at the edges of its launch shapes, against the oracle's
 token-by-token loop: append and attention in one launch (one, two and four
 key tiles a workgroup; several workgroups to a query tile), the planes'
-kernel with 1, 2, 3 and 5 workgroups to a query tile, head groups of 1, 2 and
+kernel with 1 to 8 workgroups to a query tile, head groups of 1, 2 and
 4; and buffers that overlap.
 
 Tolerance: as test_gpu_prefill.py (1e-4 on outputs; cache bit-exact).  The
@@ -25,8 +25,8 @@ SHAPES = [
     (1, 32, 4, 0, 129), (1, 32, 4, 477, 3), (1, 32, 4, 900, 120), (1, 12, 1, 200, 40), (2, 32, 4, 0, 256),
     # head groups of one and two
     (1, 8, 8, 0, 20), (1, 8, 8, 130, 5), (1, 4, 2, 40, 100), (1, 8, 4, 300, 70),
-    # planes: 5, 3, 2 and 1 workgroups to a query tile
-    (1, 32, 4, 700, 330), (1, 8, 8, 0, 500), (2, 32, 4, 0, 300), (2, 32, 4, 100, 200), (22, 32, 4, 300, 40),
+    # planes: 8, 4, 6, 5, 3, 2 and 1 workgroups to a query tile
+    (1, 32, 4, 1500, 100), (1, 32, 4, 1000, 256), (1, 32, 4, 700, 300), (1, 32, 4, 700, 330), (1, 8, 8, 0, 500), (2, 32, 4, 0, 300), (2, 32, 4, 100, 200), (22, 32, 4, 300, 40),
     (22, 32, 4, 477, 3), (22, 16, 2, 200, 220),
 ]
 

@@ -972,23 +972,32 @@ hipError_t launch_prefill_short(const PrefillParams& p, float* part, int* counte
 // Workgroups per query tile of the planes' kernel, by the launch's query tiles
 // (units: of a kv head's group of four q heads) per CU: a launch that leaves
 // CUs idle, or has one or two workgroups on each, takes the longest walk's
-// time.  Measured, us per call with 1 / 2 / 3 / 4 / 5 workgroups:
-//   88 units (one layer of 32/4 heads, 333 tokens after 1500) 97.7 / 59.3 /
-//     52.0 / 46.6 / 43.1;
-//   160 (640 tokens) 40.7 / 30.4 / 27.1 / 29.3 / 30.3; 256 (1024 tokens)
+// time.  Few units: as many workgroups as the CUs take one each, or two each
+// where one would leave every walk a third of the keys or more; a workgroup more than
+// that and some CUs hold one too many.  Measured, us per call by workgroups per
+// query tile:
+//   32 units (one layer of 32/4 heads, 128 tokens after 1900), 4 .. 10: 39.6 /
+//     35.9 / 33.5 / 33.0 / 31.8 (256 workgroups) / 36.3 / 35.8;
+//   64 (256 tokens after 1000), 3 .. 9: 35.4 / 31.0 (256) / 33.5 / 32.2 / 33.2 /
+//     33.6 (512) / 37.6;
+//   88 (333 tokens after 1500), 1 .. 6: 97.7 / 59.7 / 53.0 / 48.0 / 44.2 (440) /
+//     48.9; 96 (384 after 900), 4 .. 6: 38.7 / 36.8 (480) / 39.9;
+//   160 (640 tokens), 1 .. 4: 40.5 / 30.0 / 27.4 / 30.0; 256 (1024 tokens), 1 .. 5
 //     61.1 / 42.7 / 41.3 / 44.5 / 45.3;
-//   352 (two layers, 700 tokens) 47.9 / 39.9 / 41.9; 352 of few key tiles (22
-//     layers, 40 tokens after 140) 30.6 / 29.8 / 35.1;
-//   616 (22 layers of 16/2 heads, 429 tokens) 71.4 / 78.2.
+//   352 (two layers, 700 tokens), 1 .. 3: 47.9 / 39.9 / 41.9; 352 of few key
+//     tiles (22 layers, 40 tokens after 140) 30.6 / 29.8 / 35.1;
+//   616 (22 layers of 16/2 heads, 429 tokens), 1 / 2: 71.4 / 78.2.
 // Two key splits in each workgroup, merged in LDS (one workgroup per CU), took
-// 62.0, 28.1 and 46.3 us for the first three.
+// 62.0, 28.1 and 46.3 us for 88, 160 and 256 units; two layers of 288 to 300 tokens
+// (144 to 160 units of few key tiles), 20.5 and 21.5 us so, take 21.3 and 22.3.
 namespace {
 
 int attention_chunks(long long units, int n_kt)
 {
     const long long cus = device_cus();
-    long long n = 5 * units <= 2 * cus ? std::max<long long>(5, (cus / units) | 1)
-                  : units <= cus       ? 3
+    long long n = 4 * units <= cus       ? cus / units
+                  : 5 * units <= 2 * cus ? 2 * cus / units
+                  : units <= cus         ? 3
                   : 4 * units <= 7 * cus ? 2
                                          : 1;
     n = std::min<long long>(n, (n_kt + 1) / 2);  // two key tiles each, as the kernel does
