@@ -438,7 +438,7 @@ def test_prefill_forward_matches_token_loop(tla, O, W, engines, name):
     batched).  The last token's logits against the reference's (golden),
     in one call and in two calls (pos0 > 0); the KV cache against the
     token-by-token device path within 1e-4 of the largest entry (the
-    streamed products sum in another order), and the layer 0 of a prompt
+    batched products sum in another order), and the layer 0 of a prompt
     short enough for the multi-vector GEMVs (2 tokens of Q8_0 / Q4_0, else
     1) bit for bit (their sums are the token path's; the inputs are the
     embeddings in both)."""
@@ -518,8 +518,7 @@ def test_prefill_forward_errors(tla, W, engines):
 
 @pytest.mark.parametrize("name", ["q8_0", "f16_tied", "q4_0", "mixed"])
 def test_prefill_forward_long_prompt(tla, O, W, engines, name):
-    """A 48-token prompt: the batched projections as streamed products with
-    three token tiles (Q6_K matrices as split products).
+    """A 48-token prompt: the batched projections over three token tiles.
     Last token's logits against the oracle's token loop."""
     g = golden("forward.npz")
     spec, t = model_from_golden(W, g, name)
@@ -547,9 +546,8 @@ def test_prefill_forward_long_prompt(tla, O, W, engines, name):
 @pytest.mark.parametrize("name", ["q8_0", "f16_tied", "q4_0", "f32", "mixed"])
 def test_prefill_forward_streamed_prompt(tla, O, W, engines, name):
     """A 32-token prompt, in one call and as two calls of 16 (the second at
-    pos0 = 16): every batched projection as the streamed product (weights
-    dequantised in registers; Q/K/V as one product of three segments where
-    their formats agree).  Last token's logits and the K cache against the
+    pos0 = 16): batched projections of one and two token tiles (Q/K/V as one
+    product of three segments where their formats agree).  Last token's logits and the K cache against the
     oracle's token loop."""
     g = golden("forward.npz")
     spec, t = model_from_golden(W, g, name)

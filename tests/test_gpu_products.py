@@ -18,12 +18,12 @@ pytestmark = pytest.mark.gpu
 TYPES = [(Q.F32, "f32"), (Q.F16, "f16"), (Q.Q4_0, "q4_0"), (Q.Q8_0, "q8_0"), (Q.Q6_K, "q6_k")]
 # direct: one token tile, remainders of rows and waves, groups of four blocks
 # that the row does not fill; resident: shares of the tiles, K slices of 4 and
-# 8 blocks, two K ranges with an uneven last one; tiled (F32 and F16 first): one
-# and several K ranges, token and row remainders
+# 8 blocks, two K ranges with an uneven last one; tiled (past 64 tokens): one and
+# several K ranges, token and row remainders
 SHAPES = [(17, 64, 3), (40, 192, 4), (4112, 1088, 2), (300, 3136, 4), (300, 3136, 5), (9000, 1344, 8),
           (50, 2368, 3), (33, 256, 6), (33, 320, 8), (4112, 256, 16), (9000, 512, 15), (4112, 1024, 17),
           (4200, 2048, 33), (8200, 320, 40), (2064, 4352, 50), (4112, 2560, 193), (8208, 256, 250),
-          (6160, 1024, 100), (3000, 4096, 300)]
+          (6160, 1024, 100), (3000, 4096, 300), (8200, 576, 250)]
 
 
 def rows_close(got, raw, x, t, rows, cols, tol, what):
@@ -67,7 +67,7 @@ def test_product_infinities(W, engines, t, name, n, rows):
 # where the tiled product runs: F16 and F32 in one K range, every format but
 # Q6_K (which keeps the resident one) in several
 @pytest.mark.parametrize("t,name", TYPES)
-@pytest.mark.parametrize("n,rows,cols", [(250, 8208, 256), (300, 2064, 4352)])
+@pytest.mark.parametrize("n,rows,cols", [(250, 8208, 512), (300, 2064, 4352)])
 def test_product_infinities_many_tokens(W, engines, t, name, n, rows, cols):
     infinities(W, engines(1, 64), t, name, n, rows, cols)
 

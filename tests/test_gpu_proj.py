@@ -215,18 +215,15 @@ def test_projection_errors(tla, W, engines):
 
 BATCH_SHAPES = [(32, 256, 16), (2560, 2048, 33), (64, 5632, 128), (5632, 2048, 130), (96, 512, 300),
                 (2048, 2048, 256), (40, 5632, 257), (48, 256, 7), (40, 512, 20), (48, 256, 2)]
-# (48, 256, 2): GEMV groups (streamed for F16 / F32); (48, 256, 7), (32, 256, 16), (40, 512, 20):
-# streamed products
+# (48, 256, 2): GEMV groups (a split product for F16 / F32)
 
 
 @pytest.mark.parametrize("t,name", TYPES)
 @pytest.mark.parametrize("rows,cols,n_tok", BATCH_SHAPES)
 def test_matmul_batch(O, W, engines, t, name, rows, cols, n_tok):
     """tla_matmul_batch: groups of GEMVs (under 3 tokens, F16 / F32 under 2,
-    Q6_K under 16), the streamed product (up to 64 tokens, weights
-    dequantised in registers) or the split product (bf16 pieces of x and of
-    the weights on the matrix cores, fp32 sums), per token against the
-    oracle's matmul."""
+    Q6_K under 6) or the split products (bf16 pieces of x and of the weights
+    on the matrix cores, fp32 sums), per token against the oracle's matmul."""
     if t == Q.Q6_K and cols % 256:
         pytest.skip("Q6_K rows are whole 256-weight super-blocks")
     eng = engines(1, 64)
@@ -251,18 +248,16 @@ STREAM_SHAPES = [(2560, 2048, 16), (2048, 5632, 32), (40, 64, 17), (200, 128, 31
 @pytest.mark.parametrize("t,name", TYPES)
 @pytest.mark.parametrize("rows,cols,n_tok", STREAM_SHAPES)
 def test_matmul_batch_streamed(tla, O, W, engines, t, name, rows, cols, n_tok):
-    """The streamed product (2 or 3 to 64 tokens): rows not a multiple of its
-    16-row tiles, rows of 2 blocks (two of its four waves idle), token counts
-    not a multiple of 16, 57 and 64 tokens (four token tiles) and 65 tokens
-    (the split product past the bound); every token against the oracle's
-    matmul, and the same bits with one to four token tiles per workgroup
-    (Q6_K takes the GEMVs under 16 tokens, the split product from 16)."""
+    """2 to 65 tokens: rows not a multiple of the 16-row tiles, rows of 2 blocks
+    (most of a workgroup's waves idle), token counts not a multiple of 16;
+    every token against the oracle's matmul, and the same bits with one to
+    four token tiles per workgroup."""
     if t == Q.Q6_K and cols % 256:
         pytest.skip("Q6_K rows are whole 256-weight super-blocks")
     eng = engines(1, 64)
     raw = W.make_weights(t, rows, cols, salt=rows + 5 * cols)
     x = np.random.default_rng(n_tok + 1).standard_normal((n_tok, cols)).astype(np.float32)
-    log(f"  streamed product {name} {rows}x{cols}, {n_tok} tokens")
+    log(f"  product {name} {rows}x{cols}, {n_tok} tokens")
     outs = []
     with device_arrays() as track:
         w = track(eng.array(raw))
@@ -294,9 +289,8 @@ def test_stream_tiles_option(tla, engines):
 
 
 def test_matmul_batch_many_shapes(O, W, engines):
-    """Q6_K products of every batch size from 16 to 275 in a row on an engine
-    of its own (the split product from 16 vectors), so that the split-x and
-    partial-sum workspaces grow while products are queued; products at
+    """Q6_K products of few rows and every batch size from 16 to 275 in a row
+    on an engine of its own (direct products: no workspace); products at
     several sizes against the oracle's matmul."""
     eng = engines(1, 96)  # a key no other test uses: the workspaces start empty
     rows, cols, t = 32, 256, Q.Q6_K
@@ -315,13 +309,34 @@ def test_matmul_batch_many_shapes(O, W, engines):
                                f"{n_tok} tokens, token {i}")
 
 
+def test_matmul_batch_growing_workspaces(O, W, engines):
+    """Q8_0 products of K in several ranges and more vectors from call to call
+    on an engine of its own, so that the split-x and partial-sum workspaces
+    grow while products are queued; every product's last vector against the
+    oracle's matmul."""
+    eng = engines(1, 104)  # a key no other test uses: the workspaces start empty
+    rows, cols, t = 1040, 4352, Q.Q8_0
+    raw = W.make_weights(t, rows, cols, salt=12)
+    x = np.random.default_rng(261).standard_normal((200, cols)).astype(np.float32)
+    sizes = list(range(65, 200, 15))
+    with device_arrays() as track:
+        w, xd = track(eng.array(raw)), track(eng.array(x))
+        outs = [track(eng.array((n_tok, rows))) for n_tok in sizes]
+        for n_tok, out in zip(sizes, outs):
+            eng.matmul_batch(out.ptr, w.ptr, xd.ptr, rows, cols, n_tok, t)
+        got = [out.download() for out in outs]
+    for n_tok, o in zip(sizes, got):
+        i = n_tok - 1
+        check_rows(o[i], O.matmul(raw, x[i], rows, cols, t), raw, x[i], t, rows, cols, f"{n_tok} tokens, last")
+
+
 SPLIT_SHAPES = [(2048, 5632, 130), (2560, 2048, 65), (11264, 2048, 100), (40, 512, 70), (300, 256, 128)]
 
 
 @pytest.mark.parametrize("t,name", TYPES)
 @pytest.mark.parametrize("rows,cols,n_tok", SPLIT_SHAPES)
 def test_split_product_tilings(tla, O, W, engines, t, name, rows, cols, n_tok):
-    """The split product with 1, 2 and 4 row subtiles per wave (K in 3
+    """The split products with 1, 2 and 4 row subtiles (K in 3
     ranges) gives the same bits: every output is one wave's sums in the same
     order.  K cut into 1, 3 and 7 ranges (sums added in range order by the
     second launch), and the per-shape choice, each within the oracle bound

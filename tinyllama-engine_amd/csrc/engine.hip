@@ -823,7 +823,7 @@ int norm_product(tla_engine* e, int type, const GemvSegment* segs, int n_seg, in
 // writes the planes of silu(gate) * up, where rows are whole blocks): unless the
 // tiled product, which does not pair, is faster by more than the launch that
 // then writes the planes, less what the epilogue costs (F16, 5632 columns, a layer
-// step paired / not: 64 tokens 102.5 / 99.7 us, 96 120.4 / 129, 120 137 / 132.5).
+// step paired / not: 96 tokens 120.4 / 129 us, 120 137 / 132.5).
 // By the shape, not the options.
 bool paired_product(tla_engine* e, int type, int n_ff, int cols, int n)
 {

@@ -41,7 +41,7 @@
 //             x split (and normalised) by the workgroup itself;
 //   resident  more tokens: a workgroup keeps its rows' decoded weights in
 //             registers and streams the x planes of all token tiles past them;
-//   tiled     where its estimated time is less (many tokens; weights of several
+//   tiled     past 64 tokens, where its estimated time is less (weights of several
 //             pieces, of which the registers hold few rows; several K ranges): a
 //             64 kRW row x 64 token tile per workgroup, x through LDS.
 // Every output is a sum in a fixed order, which the shape, the CU count and
@@ -594,8 +594,9 @@ __device__ __forceinline__ void store_gated(const ProductParams& p, float sum, i
 // kR row subtiles x one token tile per workgroup, K over its 8 waves (wave w
 // blocks w, w + 8, ...; the waves' sums meet in LDS in wave order).  Every
 // load a wave makes for 2048 columns is in flight at once: the launch is one
-// memory round trip, then vector work (splitting x, about 44 operations a
-// block, and dequantising, about 30 a subtile) that bounds it.  With kXNormRows x is
+// memory round trip and the vector work after it (splitting x, about 44 operations a
+// block, and dequantising, about 30 a subtile; counters: vector units active 27-35
+// % of the busy cycles, matrix cores 4-7 %, the rest waits).  With kXNormRows x is
 // multiplied by the norm's weights before it is split and the sums by the
 // row's 1 / rms at the end, so that no launch goes before it.  Q8_0, 12
 // tokens, TinyLlama's layer (kernel trace): rmsnorm + Q/K/V 11.4 us, W_o 8.8,
@@ -827,9 +828,11 @@ __global__ __launch_bounds__(kWaves * 64) void direct_product_kernel(const Produ
 // weights are read and dequantised once per share, and nothing but the planes
 // moves per tile.  Each wave keeps kRing blocks of x ahead in registers; the
 // waves' sums meet in LDS.  Bound by the planes' way into the CU: a tile is 196 KB per
-// workgroup, 1.6 us at the ~50 B a clock a CU takes from L2, against 0.96 us of
-// matrix work with three subtiles (measured per tile: 1.77 / 1.94 / 2.1 us with 1 / 2
-// / 3 subtiles).  All workgroups walk their tiles in the same order, so an
+// workgroup, against 0.96 us of matrix work with three subtiles (measured per tile:
+// 1.77 / 1.94 / 2.1 us with 1 / 2 / 3 subtiles in short launches, 46 to 39 B a clock;
+// 33 over 512 tokens, where counters show the matrix cores busy 38 % and the vector
+// units 41 % of the time, waves waiting for loads for the rest; L2 hits 93 %).  All
+// workgroups walk their tiles in the same order, so an
 // XCD's share of them meets in its L2; a flat split of (group, tile) units over
 // the CUs did not (4 us a tile).  An LDS ring filled by direct loads was slower
 // (1.5 us + 0.31 a subtile: written and read, x passes the LDS port twice), and
@@ -987,7 +990,10 @@ __global__ __launch_bounds__(kWaves * 64) void resident_product_kernel(const Pro
 // wave w owns rows 16 kRW w .. + 16 kRW - 1 for all 64 tokens.  The x blocks
 // pass through a ring of three LDS stages (12 KiB each) filled by direct
 // loads two blocks ahead; each wave loads its rows' weights three blocks
-// ahead.  Bound by its barrier per block and LDS reads.  Carrying the sums
+// ahead.  Bound by the barrier per block between short stretches of decoding, LDS
+// reads and products: neither unit is the limit (counters, 512 tokens: Q4_0 2048 x
+// 5632 matrix cores busy 35 %, vector units 55 %; F16 5632 x 2048 51 / 53 %), and
+// every XCD reads all the weights.  Carrying the sums
 // of types without a scale through the matrix cores was 3-6 % faster and put a
 // layer of F16 over 100 sequences 3.6e-7 off fp64 against 1.4e-7.
 template <int kType, int kRW>
@@ -1435,17 +1441,20 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         return;
     }
     // Resident or tiled by the shape's estimates (the options change no kind).
-    // Of 971 shapes measured in both kernels (F16, F32, Q4_0, Q8_0; 512 to 32000
-    // rows, 512 to 8192 columns, 20 to 1000 tokens) this takes the slower one by
-    // more than 5 % in 32 (lines of rows and tokens fitted to 2048 columns: 224),
-    // 0.4 % on average (4 %).  Us, resident / tiled: F16 8192 x 2048, 81 tokens
+    // Of 838 shapes measured in both kernels (F16, F32, Q4_0, Q8_0; 512 to 32000
+    // rows, 512 to 8192 columns, 65 to 1000 tokens) this takes the slower one by
+    // more than 5 % in 30 (lines of rows and tokens fitted to 2048 columns: 153),
+    // 0.5 % on average (2.5 %).  Us, resident / tiled: F16 8192 x 2048, 81 tokens
     // 25.4 / 34.9, 11264 x 2048, 128 tokens 53.1 / 45.8, 8192 x 1024, 128 18.7 /
     // 26.4; F32 4096 x 2048, 160 31.6 / 35.8, 2048 x 5632, 65 38.3 / 33.9; Q8_0
-    // 4096 x 5632, 128 46.1 / 40.6, 2048 x 4096, 256 34.3 / 35.1.  Neither a pair's
-    // epilogue nor Q6_K's decoding is in the tiled kernel.
+    // 4096 x 5632, 128 46.1 / 40.6, 2048 x 4096, 256 34.3 / 35.1.
+    // Up to one column of 64 tokens the resident product stays, for its shorter
+    // chains of sums (F16 11264 x 2048, 56 tokens: 1.00e-7 off fp64 in 33.1 us,
+    // tiled 1.07e-7 in 28.9), and below 512 columns, where neither was measured.
+    // Neither a pair's epilogue nor Q6_K's decoding is in the tiled kernel.
     ProductParams tiled = *p;
     plan_resident(type, n_cu, 0, 0, 0, p);
-    if (!p->pair && type != kQ6_K) {
+    if (!p->pair && type != kQ6_K && p->n > 16 * kTW && n_blk >= 16) {
         plan_tiled(n_cu, 0, 0, &tiled);
         if (product_us(type, n_cu, tiled) < product_us(type, n_cu, *p)) {
             *p = tiled;
