@@ -233,10 +233,14 @@ int tla_matmul(tla_engine* e, float* out_dev, const void* w_dev, const float* x_
  * registers into exact bf16 pieces, every product of pieces exact in the fp32
  * accumulator of the bf16 matrix cores; up to 16 vectors, or for few rows,
  * x is split by the product itself, else by a launch before it into an engine
- * workspace of 6 bytes per element (tokens padded to 64), and rows of more than
- * 2048 columns are cut into ranges whose sums are added in order from a
- * second workspace.  Fewer vectors run as groups of matrix-vector products.
- * fp32 accumulation throughout: equal to the reference to fp32 rounding.
+ * workspace of 6 bytes per element (vectors padded to 64), and K may be cut into
+ * ranges (always past 2048 columns; where it fills the GPU, also shorter rows)
+ * whose sums are added in order from a second workspace of 4 bytes per vector,
+ * row and range.  The workspaces grow on demand (after a stream synchronize) and
+ * are kept.  Fewer vectors run as groups of matrix-vector products.
+ * fp32 accumulation throughout: equal to the reference to fp32 rounding, and
+ * what fp32 gives for infinities and NaNs (one such vector costs the batch 10 to
+ * 50 % with a NaN, several times its time with an infinity).
  * Used for the prompt's projections and a layer over several sequences. */
 int tla_matmul_batch(tla_engine* e, float* out_dev, const void* w_dev, const float* x_dev, int rows,
                      int cols, int n_tok, int type);
@@ -251,9 +255,9 @@ int tla_vec_add(tla_engine* e, float* out_dev, const float* x_dev, int size);
 /* The input half of the attention block for n_seq sequences
  * (src/forward.cpp:180-190): xb = rmsnorm(x, norm_w, eps) (skipped when
  * norm_w is NULL), q = Wq.xb, k = Wk.xb, v = Wv.xb: one launch for one or two
- * sequences, from 3 (F16 and F32 2, Q6_K 8; x and norm_w 16-byte aligned) the
- * products of tla_matmul_batch, else one launch per 8 sequences (fewer when
- * 8 x n_embd floats exceed 60 KiB).  x, q [n_seq][n_embd];
+ * sequences, from 3 (F16 and F32 2, Q6_K 6; x and norm_w 16-byte aligned) the
+ * products of tla_matmul_batch with its workspaces, else one launch per 8
+ * sequences (fewer when 8 x n_embd floats exceed 60 KiB).  x, q [n_seq][n_embd];
  * k, v [n_seq][kv_dim]; Wq [n_embd][n_embd],
  * Wk, Wv [kv_dim][n_embd], all of one type.  q and k leave unrotated, ready
  * for tla_decode with TLA_ROTATE (RoPE and the cache append are its
@@ -263,7 +267,8 @@ int tla_attn_qkv(tla_engine* e, int n_seq, float* q_dev, float* k_dev, float* v_
                  const void* wk_dev, const void* wv_dev, int type);
 
 /* The output half (src/forward.cpp:210-213): x += Wo . xb2 for n_seq
- * sequences, x and xb2 [n_seq][n_embd], Wo [n_embd][n_embd]. */
+ * sequences, x and xb2 [n_seq][n_embd], Wo [n_embd][n_embd]; from 3 (F16 and
+ * F32 2, Q6_K 6) as the product of tla_matmul_batch with its workspaces. */
 int tla_attn_out(tla_engine* e, int n_seq, float* x_dev, const void* wo_dev,
                  const float* xb2_dev, int type);
 
@@ -286,7 +291,8 @@ int tla_ffn_swiglu(tla_engine* e, float* out_dev, const float* in_dev, float* hb
 /* The FFN half of a layer (src/forward.cpp:215-228) for n_seq sequences:
  * x += ffn_swiglu(rmsnorm(x, norm_w, eps)): rmsnorm + gate and up
  * projections, then SiLU, gating, down projection and the residual add (from
- * 3 sequences, F16 and F32 2, Q6_K 8, as the products of tla_matmul_batch).
+ * 3 sequences, F16 and F32 2, Q6_K 6, as the products of tla_matmul_batch, with
+ * its workspaces and another like the first for n_ff columns).
  * x [n_seq][n_embd]; hb_dev scratch [n_seq][2][n_ff] receives the raw gate
  * and up projections, except for one sequence of Q8_0 / Q4_0 / Q6_K weights
  * (n_embd <= 4096, n_ff even): then the gate half receives SiLU(gate) x up,
@@ -364,8 +370,10 @@ int tla_forward(tla_engine* e, const tla_model* m, float* key_cache_dev, float* 
  * after n_tok forward() calls (to fp32 rounding: the attention sums are
  * grouped differently).  Engine memory it keeps for later calls: the split
  * product's workspaces, 6 bytes per token (padded to 64) and column of the
- * widest product inputs, n_embd and n_ff (TinyLlama, 512 tokens: 24 MB), and
- * partial sums of 4 bytes per token, row and 2048 columns of W_down (12 MB). */
+ * widest product inputs, n_embd and n_ff (TinyLlama, 512 tokens: 24 MB),
+ * partial sums of 4 bytes per token, row and K range of its products (up to 18
+ * ranges of a few tokens; 512 tokens: 5 of W_down, 21 MB), and what tla_prefill
+ * keeps for one layer. */
 int tla_prefill_forward(tla_engine* e, const tla_model* m, float* key_cache_dev,
                         float* value_cache_dev, const int* tokens_host, int n_tok, int pos0,
                         float* logits_dev);
@@ -391,8 +399,9 @@ enum tla_kernel_id {
     TLA_KERNEL_DECODE = 0,  /* split-KV decode attention (and forward()'s
                                short-context attention + W_o): RoPE + append +
                                attention + split merge, one launch           */
-    TLA_KERNEL_PREFILL = 1, /* causal MFMA prefill attention                 */
-    TLA_KERNEL_APPEND = 2,  /* prefill RoPE + cache append                   */
+    TLA_KERNEL_PREFILL = 1, /* causal MFMA prefill attention (short prompts: with
+                               their RoPE + append, one launch)              */
+    TLA_KERNEL_APPEND = 2,  /* prefill RoPE + cache append, as its own launch */
     TLA_KERNEL_GEMV = 3,    /* projections: matmul / attn_qkv / attn_out /
                                ffn / classifier                              */
     TLA_KERNEL_COUNT = 4
