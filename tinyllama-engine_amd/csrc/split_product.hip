@@ -1389,24 +1389,28 @@ void plan_tiled(int n_cu, int opt_rows, int opt_k, ProductParams* p)
 
 }  // namespace
 
-// Resident: as in plan_resident, a tile's time by its columns and by the piece
-// products per multiply-add.  Tiled: a block of a workgroup takes 0.3 where its CU
-// has no other, else the CU's workgroups share its matrix cores and LDS.  Several
-// ranges: the launch that adds their sums, a step per range, and its bytes.
+// Fitted to both kernels' times at 992 shapes (plan_product), within 6 %.
+// Resident: per round of workgroups the weights of a row subtile (2.6 at 2048
+// columns) and each token tile, whose planes and products overlap in part; a wave
+// loads a slice of 4 or 8 blocks of it, used or not.  Tiled: a block of a
+// workgroup takes 0.23 where its CU has no other, else the CU's workgroups share
+// its matrix cores, vector units and LDS.  Several ranges: the launch that adds
+// their sums, a step per range, and its bytes.
 double product_us(int type, int n_cu, const ProductParams& p)
 {
-    const int products = type == kF32 ? 6 : type == kF16 || type == kQ6_K ? 5 : 3;
-    const double sums = p.k_splits > 1 ? 3.5 + 0.3 * p.k_splits + 0.8e-6 * p.n * p.total_rows * (p.k_splits + 1.0) : 0;
+    const double sums = p.k_splits > 1 ? 1.85 + 0.26 * p.k_splits + 1e-6 * p.n * p.total_rows * (p.k_splits + 1.0) : 0;
     const auto rounds = [&](long long groups) { return static_cast<double>((groups + n_cu - 1) / n_cu); };
     const int r = p.rows_per_group;
     if (p.kind == kProductTiled) {
-        const double block = type == kF32 ? 0.36 * r : type == kF16 ? 0.26 * r : 0.08 + 0.18 * r;
+        const double block = type == kF32 ? 0.372 * r : type == kF16 ? 0.257 * r : 0.05 + 0.184 * r;
         const double per_cu = rounds(static_cast<long long>(p.row_groups) * (p.n_tiles / kTW) * p.k_splits);
-        return sums + 5 + p.blk_per_split * std::max(0.3, per_cu * block);
+        return sums + 3.7 + 0.33 * per_cu + p.blk_per_split * std::max(0.23, per_cu * block);
     }
     const int each = (p.n_tiles + p.shares - 1) / p.shares;
-    const double tile = (1.6 + 0.085 * products * r) * p.blk_per_split / kRangeBlocks;
-    return sums + rounds(static_cast<long long>(p.row_groups) * p.k_splits * p.shares) * (3.0 + 1.5 * r + each * tile);
+    const double slice = p.blk_per_split <= 4 * kWaves ? 0.5 : 1.0;
+    const double tile = (0.9 + (type == kF32 ? 1.18 : type == kF16 || type == kQ6_K ? 0.54 : 0.4) * r) * slice;
+    return sums + rounds(static_cast<long long>(p.row_groups) * p.k_splits * p.shares) *
+                      (1.7 + 2.6 * r * p.blk_per_split / kRangeBlocks + each * tile);
 }
 
 void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, ProductParams* p)
@@ -1441,20 +1445,21 @@ void plan_product(int type, int n_cu, int opt_rows, int opt_tiles, int opt_k, Pr
         return;
     }
     // Resident or tiled by the shape's estimates (the options change no kind).
-    // Of 838 shapes measured in both kernels (F16, F32, Q4_0, Q8_0; 512 to 32000
-    // rows, 512 to 8192 columns, 65 to 1000 tokens) this takes the slower one by
-    // more than 5 % in 30 (lines of rows and tokens fitted to 2048 columns: 153),
-    // 0.5 % on average (2.5 %).  Us, resident / tiled: F16 8192 x 2048, 81 tokens
+    // Of 992 shapes measured in both kernels (F16, F32, Q4_0, Q8_0; 512 to 32000
+    // rows, 256 to 8192 columns, 65 to 1000 tokens) this takes the slower one by
+    // more than 5 % in 20 (lines of rows and tokens fitted to 2048 columns: 178),
+    // 0.3 % on average (2.5 %).  Us, resident / tiled: F16 8192 x 2048, 81 tokens
     // 25.4 / 34.9, 11264 x 2048, 128 tokens 53.1 / 45.8, 8192 x 1024, 128 18.7 /
     // 26.4; F32 4096 x 2048, 160 31.6 / 35.8, 2048 x 5632, 65 38.3 / 33.9; Q8_0
-    // 4096 x 5632, 128 46.1 / 40.6, 2048 x 4096, 256 34.3 / 35.1.
+    // 4096 x 5632, 128 46.1 / 40.6, 2048 x 4096, 256 34.3 / 35.1; F32 3000 x 256, 512
+    // tokens 34.8 / 17.2.
     // Up to one column of 64 tokens the resident product stays, for its shorter
     // chains of sums (F16 11264 x 2048, 56 tokens: 1.00e-7 off fp64 in 33.1 us,
-    // tiled 1.07e-7 in 28.9), and below 512 columns, where neither was measured.
+    // tiled 1.07e-7 in 28.9).
     // Neither a pair's epilogue nor Q6_K's decoding is in the tiled kernel.
     ProductParams tiled = *p;
     plan_resident(type, n_cu, 0, 0, 0, p);
-    if (!p->pair && type != kQ6_K && p->n > 16 * kTW && n_blk >= 16) {
+    if (!p->pair && type != kQ6_K && p->n > 16 * kTW) {
         plan_tiled(n_cu, 0, 0, &tiled);
         if (product_us(type, n_cu, tiled) < product_us(type, n_cu, *p)) {
             *p = tiled;
